@@ -846,9 +846,12 @@ int launch_visc(sifv_handle* h, int src, const int* active) {
     A.sigma = h->cfg.surfaceTensionSigma;
     A.capEps = h->cfg.surfaceTensionEps;
     A.out = h->visc;
+    const int tx = h->dim >= 2 ? kViscCols : 256;
+    const long nblk = (long)((h->nx + tx - 1) / tx) * (h->dim >= 2 ? (h->ny + kViscRows - 1) / kViscRows : 1) *
+                      (h->dim == 3 ? (h->nz + kViscPlanes - 1) / kViscPlanes : 1);
     void* args[] = {&A};
-    HIPCHK(hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3(elementwise_blocks(h)), dim3(256), args, 0,
-                           h->stream));
+    HIPCHK(hipLaunchKernel(reinterpret_cast<const void*>(fn), dim3((unsigned)nblk),
+                           dim3(h->dim >= 2 ? kViscCols * kViscRows : 256), args, 0, h->stream));
     return SIFV_OK;
 }
 
