@@ -14,8 +14,12 @@
 // Work decomposition (wave64).  1D/2D (`stage_xy_kernel`, MODE_FULL): one
 // wave owns a strip of 62 consecutive columns plus one halo column on each
 // side (lane l <-> column X0-1+l) and marches upward through `rows` rows.
-// The y-stencil of each lane's column lives in a register window that slides
-// one row per iteration; the x-stencil is exchanged through LDS.  Each lane
+// The y-stencil of each lane's column is the R rows above the current one in
+// registers, sliding one row per iteration, and the current row and the one
+// below it in LDS, where the x-stencil of the current row is read anyway.
+// (All rows in registers took 176 VGPRs, one wave per SIMD fewer or spills;
+// spilled registers cost HBM traffic.  4096^2 FP64: 843 -> 758 us per launch
+// together with weno5_set and row addressing, same box.)  Each lane
 // reconstructs its own cell once per direction (both face states from one
 // stencil), so every face flux is computed once per strip.
 // 3D: the same kernel runs on each z-plane (MODE_XY) and writes the x+y part
@@ -309,13 +313,78 @@ __device__ __forceinline__ void load_raw(const StageParams<T>& P, const T* buf, 
     rc.flip = fl;
 }
 
+// A cell as a wave-uniform row (element offset of the row's first padded cell)
+// plus a per-lane column: the address of a field's value is then a scalar base
+// and one 32-bit vector offset shared by all fields, with no 64-bit vector
+// arithmetic per access.
+struct RowRef {
+    size_t row;    // uniform
+    unsigned c;    // padded column, i + ngx
+};
+template <typename A>
+__device__ __forceinline__ A* field_at(A* base, size_t total, int q, size_t id) {
+    return base + (size_t)q * total + id;
+}
+template <typename A>
+__device__ __forceinline__ A* field_at(A* base, size_t total, int q, const RowRef& r) {
+    const unsigned off = r.c * (unsigned)sizeof(A);
+    return reinterpret_cast<A*>(reinterpret_cast<uintptr_t>(base + ((size_t)q * total + r.row)) + off);
+}
+__device__ __forceinline__ size_t row_base(const Grid& g, int j, int k) {
+    return (size_t)g.nxT * ((size_t)(j + g.ngy) + (size_t)g.nyT * (size_t)(k + g.ngz));
+}
+// Sign flips of the velocity components by one axis' ghost rule (bit d: u[d]).
+__device__ __forceinline__ unsigned flip_mask(int axis, bool fn, bool ft) {
+    return (fn ? 1u << axis : 0u) ^ (ft ? 7u & ~(1u << axis) : 0u);
+}
+
+// Raw values of the cell in column cm (mapped column and its flips) of row j,
+// plane k through the ghost mapping; j and k are wave-uniform.
+struct ColMap {
+    unsigned c, flip;
+};
+__device__ __forceinline__ ColMap map_column(const Grid& g, int i) {
+    bool fn = false, ft = false;
+    const int si = map_axis(clampi(i, -g.ngx, g.nx - 1 + g.ngx), g.nx, g.bc[0], g.bc[1], fn, ft);
+    return ColMap{(unsigned)(si + g.ngx), flip_mask(0, fn, ft)};
+}
+template <int DIM, int NPH, typename T>
+__device__ __forceinline__ void load_row(const StageParams<T>& P, const T* buf, const ColMap& cm, int j, int k,
+                                         RawCell<DIM, NPH, T>& rc) {
+    constexpr int NCV = DIM + 2 + 2 * NPH;
+    const Grid& g = P.g;
+    unsigned fl = cm.flip;
+    int sj = j, sk = k;
+    if (DIM >= 2 && (j < 0 || j >= g.ny)) {
+        bool fn = false, ft = false;
+        sj = map_axis(clampi(j, -g.ngy, g.ny - 1 + g.ngy), g.ny, g.bc[2], g.bc[3], fn, ft);
+        fl ^= flip_mask(1, fn, ft);
+    }
+    if (DIM >= 3 && (k < 0 || k >= g.nz)) {
+        bool fn = false, ft = false;
+        sk = map_axis(clampi(k, -g.ngz, g.nz - 1 + g.ngz), g.nz, g.bc[4], g.bc[5], fn, ft);
+        fl ^= flip_mask(2, fn, ft);
+    }
+    const RowRef r{row_base(g, DIM >= 2 ? sj : 0, DIM >= 3 ? sk : 0), cm.c};
+#pragma unroll
+    for (int q = 0; q < NCV; ++q) rc.U[q] = *field_at(buf, P.total, q, r);
+    rc.flip = fl;
+}
+
+// u with its sign flipped when bit d of the flips is set.
+__device__ __forceinline__ double flip_sign(double u, unsigned flip, int d) {
+    return __hiloint2double(__double2hiint(u) ^ (int)((flip >> d) << 31), __double2loint(u));
+}
+__device__ __forceinline__ float flip_sign(float u, unsigned flip, int d) {
+    return __int_as_float(__float_as_int(u) ^ (int)((flip >> d) << 31));
+}
+
 template <int DIM, int NPH, typename T, typename C>
 __device__ __forceinline__ void raw_to_cell(const StageParams<T>& P, const RawCell<DIM, NPH, T>& rc,
                                             Cell<DIM, NPH, C>& c) {
     convert_cell<DIM, NPH, T, C>(P.eos, P.mix, rc.U, c);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
-        if (rc.flip & (1u << d)) c.u[d] = -c.u[d];
+    for (int d = 0; d < DIM; ++d) c.u[d] = flip_sign(c.u[d], rc.flip, d);
 }
 
 // Load one cell (i, j, k) through the ghost mapping (with velocity flips).
@@ -463,8 +532,8 @@ __device__ __forceinline__ void accumulate(T* acc, const T* lo, const T* hi, T c
 
 // Body force and face stresses of one cell (src/ExplicitSolver.cpp:498-535,
 // src/SemiImplicitSolver.cpp:484-520), added to the flux part in FP64.
-template <int DIM, typename T, typename C>
-__device__ __forceinline__ void add_sources(const StageParams<T>& P, size_t id, T* acc, C rhoC, const C* uC) {
+template <int DIM, typename T, typename C, typename ID>
+__device__ __forceinline__ void add_sources(const StageParams<T>& P, ID id, T* acc, C rhoC, const C* uC) {
     if (P.bodyForce) {
         const double a[3] = {P.accel[0], P.accel[1], P.accel[2]};
         const double rho = (double)rhoC;
@@ -478,8 +547,8 @@ __device__ __forceinline__ void add_sources(const StageParams<T>& P, size_t id, 
     }
     if (P.visc) {
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) acc[1 + d] = (T)((double)acc[1 + d] + P.visc[(size_t)d * P.total + id]);
-        acc[DIM + 1] = (T)((double)acc[DIM + 1] + P.visc[(size_t)DIM * P.total + id]);
+        for (int d = 0; d < DIM; ++d) acc[1 + d] = (T)((double)acc[1 + d] + *field_at(P.visc, P.total, d, id));
+        acc[DIM + 1] = (T)((double)acc[DIM + 1] + *field_at(P.visc, P.total, DIM, id));
     }
 }
 
@@ -497,12 +566,12 @@ __device__ __forceinline__ void store_state(T* a, T v) {
     else *a = v;
 }
 
-template <int DIM, typename T, bool SRC>
-__device__ __forceinline__ double finish_cell_f32(const StageParams<T>& P, size_t id, T* acc,
+template <int DIM, typename T, bool SRC, typename ID>
+__device__ __forceinline__ double finish_cell_f32(const StageParams<T>& P, ID id, T* acc,
                                                   const Cell<DIM, 0, float>& cell, const double* h, double dt,
                                                   bool wantDt, const T* Upre, const T* U0pre) {
     constexpr int NCV = DIM + 2;
-    if (SRC) add_sources<DIM, T, float>(P, id, acc, cell.rho, cell.u);
+    if (SRC) add_sources<DIM, T, float, ID>(P, id, acc, cell.rho, cell.u);
     float un[NCV];
     const bool use0 = P.c2 != 0.0;
     const float c1 = (float)P.c1, c2 = (float)P.c2, c3dt = (float)(P.c3 * dt);
@@ -510,13 +579,13 @@ __device__ __forceinline__ double finish_cell_f32(const StageParams<T>& P, size_
     const float dtf = (float)dt;
 #pragma unroll
     for (int q = 0; q < NCV; ++q) {
-        const float U = (float)(Upre ? Upre[q] : P.src[(size_t)q * P.total + id]);
+        const float U = (float)(Upre ? Upre[q] : *field_at(P.src, P.total, q, id));
         const float R = (float)acc[q];
         if (P.rk1) {
             un[q] = fmaf(dtf, R, U);
         } else {
             float a = c1 * U;
-            if (use0) a = fmaf(c2, (float)(U0pre ? U0pre[q] : P.u0[(size_t)q * P.total + id]), a);
+            if (use0) a = fmaf(c2, (float)(U0pre ? U0pre[q] : *field_at(P.u0, P.total, q, id)), a);
             const float b = fmaf(c3dt, R, a);
             // b / c4: exact product for c4 = 1, 2, 4; for c4 = 3 the product with
             // the rounded 1/3 is biased by +3e-8 (a drift of the whole state over
@@ -525,7 +594,7 @@ __device__ __forceinline__ double finish_cell_f32(const StageParams<T>& P, size_
             if (!P.c4pow2) qt = fmaf(fmaf(-c4, qt, b), c4i, qt);
             un[q] = qt;
         }
-        store_state<DIM>(&P.dst[(size_t)q * P.total + id], (T)un[q]);
+        store_state<DIM>(field_at(P.dst, P.total, q, id), (T)un[q]);
     }
     if (!wantDt) return 1.0e300;
     if (P.eos.stiffened) {
@@ -555,12 +624,12 @@ __device__ __forceinline__ double finish_cell_f32(const StageParams<T>& P, size_
 // SRC = false: an instantiation for configurations without body force and
 // face stresses, which carries none of their code (P.bodyForce and P.visc
 // must then be off).
-template <int DIM, int NPH, bool SEMI, typename T, bool SRC = true, typename C = double>
-__device__ __forceinline__ double finish_cell(const StageParams<T>& P, size_t id, T* acc,
+template <int DIM, int NPH, bool SEMI, typename T, bool SRC = true, typename C = double, typename ID = size_t>
+__device__ __forceinline__ double finish_cell(const StageParams<T>& P, ID id, T* acc,
                                               const Cell<DIM, NPH, C>& cell, const double* h, double dt, bool wantDt,
                                               const T* Upre = nullptr, const T* U0pre = nullptr) {
     if constexpr (sizeof(C) == 4) {
-        return finish_cell_f32<DIM, T, SRC>(P, id, acc, cell, h, dt, wantDt, Upre, U0pre);
+        return finish_cell_f32<DIM, T, SRC, ID>(P, id, acc, cell, h, dt, wantDt, Upre, U0pre);
     }
     constexpr int NCV = DIM + 2 + 2 * NPH;
     constexpr int QP = NCV, QD = NCV + 1;
@@ -569,16 +638,16 @@ __device__ __forceinline__ double finish_cell(const StageParams<T>& P, size_t id
 #pragma unroll
     for (int ph = 0; ph < NPH; ++ph) acc[DIM + 2 + NPH + ph] = acc[DIM + 2 + NPH + ph] + (T)cell.a[ph] * acc[QD];
     if constexpr (SEMI) acc[QP] = acc[QP] + (T)cell.p * acc[QD];
-    if (SRC) add_sources<DIM, T, C>(P, id, acc, cell.rho, cell.u);
+    if (SRC) add_sources<DIM, T, C, ID>(P, id, acc, cell.rho, cell.u);
     double un[NCV];
     double U0v[NCV];
     double Uv[NCV];
     const bool use0 = P.c2 != 0.0;
 #pragma unroll
     for (int q = 0; q < NCV; ++q)
-        U0v[q] = use0 ? (double)(U0pre ? U0pre[q] : P.u0[(size_t)q * P.total + id]) : 0.0;
+        U0v[q] = use0 ? (double)(U0pre ? U0pre[q] : *field_at(P.u0, P.total, q, id)) : 0.0;
 #pragma unroll
-    for (int q = 0; q < NCV; ++q) Uv[q] = (double)(Upre ? Upre[q] : P.src[(size_t)q * P.total + id]);
+    for (int q = 0; q < NCV; ++q) Uv[q] = (double)(Upre ? Upre[q] : *field_at(P.src, P.total, q, id));
     // stored energies relative to the volume fractions they were stored with:
     // the update runs on the total energies (offsets added back here and the
     // new state's offset taken off after the clamps)
@@ -629,7 +698,7 @@ __device__ __forceinline__ double finish_cell(const StageParams<T>& P, size_t id
     }
 #pragma unroll
     for (int q = 0; q < NCV; ++q)
-        if (!(SEMI && q == DIM + 1)) store_state<DIM>(&P.dst[(size_t)q * P.total + id], (T)un[q]);
+        if (!(SEMI && q == DIM + 1)) store_state<DIM>(field_at(P.dst, P.total, q, id), (T)un[q]);
     if constexpr (SEMI) {
         // advected pressure (src/SemiImplicitSolver.cpp:168,185-186); the
         // stage-0 pressure is the conversion of the backup state
@@ -640,11 +709,11 @@ __device__ __forceinline__ double finish_cell(const StageParams<T>& P, size_t id
             p0 = c0.p;
         }
         double a = P.c1 * cell.p + P.c2 * p0;
-        P.pAdv[id] = (a + (P.c3 * dt) * (double)acc[QP]) / P.c4;
-        P.pres[id] = cell.p;
+        *field_at(P.pAdv, 0, 0, id) = (a + (P.c3 * dt) * (double)acc[QP]) / P.c4;
+        *field_at(P.pres, 0, 0, id) = cell.p;
         double rs = dmax_ref(un[0], 1e-14);
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) P.vel[d][id] = un[1 + d] / rs;
+        for (int d = 0; d < DIM; ++d) *field_at(P.vel[d], 0, 0, id) = un[1 + d] / rs;
         if (P.rhoc2) {
             // rho c^2 of the updated state at the stage-start pressure, as the
             // pressure system's set-up forms it (semi_setup_kernel)
@@ -662,7 +731,7 @@ __device__ __forceinline__ double finish_cell(const StageParams<T>& P, size_t id
                 const double pinf = P.eos.stiffened ? P.eos.pInf : 0.0;
                 c = sqrt(P.eos.gamma * dmax_ref(cell.p + pinf, 1e-14) / dmax_ref(rho, 1e-14));
             }
-            P.rhoc2[id] = rho * c * c;
+            *field_at(P.rhoc2, 0, 0, id) = rho * c * c;
         }
         return 1.0e300;
     }
@@ -691,21 +760,14 @@ __device__ __forceinline__ void recon_window(const StageParams<T>& P, const Cell
                                              FaceState<DIM, NPH, T>& minusS, FaceState<DIM, NPH, T>& plusS) {
     constexpr int NV = n_recon<DIM, NPH>();
     constexpr int S = 2 * R - 1;
-    T st[S], mn[NV], pl[NV], vv[S][NV];
+    T mn[NV], pl[NV], vv[S][NV];
 #pragma unroll
     for (int s = 0; s < S; ++s) recon_vars<DIM, NPH, T>(win[first + s], vv[s]);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) st[s] = vv[s][v];
-        Recon<R, T>::run(st, eps, weno, mn[v], pl[v]);
-    }
+    recon_set<R, T, NV>([&](int v, int s) __attribute__((always_inline)) { return vv[s][v]; }, eps, weno, mn, pl);
     T sm = T(0), sl = T(0);
-    if (useSig) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) st[s] = sigwin[first + s];
-        Recon<R, T>::run(st, eps, weno, sm, sl);
-    }
+    if (useSig)
+        recon_set<R, T, 1>([&](int, int s) __attribute__((always_inline)) { return sigwin[first + s]; }, eps, weno, &sm,
+                           &sl);
     face_state<DIM, NPH, T>(P, mn, sm, minusS);
     face_state<DIM, NPH, T>(P, pl, sl, plusS);
 }
@@ -756,11 +818,8 @@ stage_xy_kernel(StageParams<T> P) {
     constexpr int NF = n_fc<DIM, NPH>();      // face contribution length
     constexpr int NFL = DIM + 4 + NPH;        // Riemann output length
     constexpr int E = R - 1;                  // extra LDS columns per side
-    constexpr int S = 2 * R - 1;              // stencil width
-    constexpr int WLO = (R >= 2) ? (2 - R) : 0;
-    constexpr int WS = R - WLO + 1;           // window rows
-    constexpr int WROW = -WLO;                // window slot of row r
-    constexpr int WST = (R >= 2) ? 0 : 1;     // first stencil slot of row r+1
+    constexpr bool kSig = RS == RS_LF;        // sigma is reconstructed (IGR)
+    constexpr int NPV = NV + (kSig ? 1 : 0);
     constexpr bool YDIR = DIM >= 2;
 
     if (P.active && *P.active == 0) return;
@@ -778,11 +837,10 @@ stage_xy_kernel(StageParams<T> P) {
     const int Y0 = YDIR ? seg * P.rows : 0;
     const int Y1 = YDIR ? ((Y0 + P.rows < g.ny) ? Y0 + P.rows : g.ny) : 1;
     const bool owned = lane >= 1 && lane <= kOwn && col < g.nx;
-    const bool useSig = (RS == RS_LF) && P.igr;
+    const bool useSig = kSig && P.igr;
     const bool incP = !SEMI;
     const bool igr = P.igr != 0;
 
-    __shared__ T sp[NV + 1][kWave + 2 * E];
 
     int ecol = 0;
     if (lane < E) ecol = X0 - 1 - E + lane;
@@ -802,33 +860,36 @@ stage_xy_kernel(StageParams<T> P) {
     const double cyU = (dxc * dzk) / ((dxc * dyU) * dzk);
 
     using C = CellT<T, NPH, SEMI>;
-    // interior fast path: when every column the wave reads (its 64 lanes and
-    // the E halo columns either side) lies inside the mesh, a load of an
-    // interior row needs no ghost mapping, clamp or velocity flip
-    const bool xin = X0 - 1 - E >= 0 && X0 + kWave - 1 + E < g.nx;
-    auto loadRaw = [&](int c, int row, RawCell<DIM, NPH, T>& rc) __attribute__((always_inline)) {
-        if (xin && row >= 0 && row < g.ny) {
-            const size_t id = cell_index(g, c, row, kz);
-#pragma unroll
-            for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) rc.U[q] = P.src[(size_t)q * P.total + id];
-            rc.flip = 0;
-        } else {
-            load_raw<DIM, NPH, T>(P, P.src, c, row, kz, rc);
-        }
+    // this lane's column, and on the first 2E lanes the halo column it loads,
+    // through the x ghost rule once for the whole march
+    const ColMap cm = map_column(g, col), em = map_column(g, E > 0 ? ecol : col);
+    auto loadRaw = [&](const ColMap& c, int row, RawCell<DIM, NPH, T>& rc) __attribute__((always_inline)) {
+        load_row<DIM, NPH, T>(P, P.src, c, row, kz, rc);
     };
-    auto loadCell = [&](int c, int row, Cell<DIM, NPH, C>& out) __attribute__((always_inline)) {
-        if (xin && row >= 0 && row < g.ny) {
-            const size_t id = cell_index(g, c, row, kz);
-            T U[DIM + 2 + 2 * NPH];
-#pragma unroll
-            for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) U[q] = P.src[(size_t)q * P.total + id];
-            convert_cell<DIM, NPH, T, C>(P.eos, P.mix, U, out);
-        } else {
-            load_cell<DIM, NPH>(P, P.src, c, row, kz, out);
-        }
+    auto loadCell = [&](const ColMap& c, int row, Cell<DIM, NPH, C>& out) __attribute__((always_inline)) {
+        RawCell<DIM, NPH, T> rc;
+        loadRaw(c, row, rc);
+        raw_to_cell<DIM, NPH, T>(P, rc, out);
     };
-    Cell<DIM, NPH, C> win[WS];
-    T sigwin[WS];
+    // primitive rows r and r-1 (by parity) of the march: the x stencil of row r
+    // and the two oldest rows of the y stencil of row r+1 (own column); sar:
+    // partial densities of row r
+    __shared__ C sp[2][NPV][kWave + 2 * E];
+    __shared__ C sar[NPH > 0 ? NPH : 1][NPH > 0 ? kWave : 1];
+    // rows r+1 .. r+R, one per register slot
+    Cell<DIM, NPH, C> win[R];
+    T sigwin[R];
+    auto putRow = [&](const Cell<DIM, NPH, C>& c, T sg, int row, int pos) __attribute__((always_inline)) {
+        C* o = &sp[row & 1][0][pos];
+        o[0] = c.rho;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) o[(1 + d) * (kWave + 2 * E)] = c.u[d];
+        o[(DIM + 1) * (kWave + 2 * E)] = c.p;
+#pragma unroll
+        for (int ph = 0; ph < NPH; ++ph) o[(DIM + 2 + ph) * (kWave + 2 * E)] = c.a[ph];
+        if constexpr (kSig) o[NV * (kWave + 2 * E)] = (C)sg;
+    };
+    auto sigAt = [&](int c, int row) { return useSig ? (T)load_sigma<DIM>(P, c, row, kz) : T(0); };
     FaceState<DIM, NPH, T> plusPrev;
     T Glo[NF];
 #pragma unroll
@@ -837,21 +898,32 @@ stage_xy_kernel(StageParams<T> P) {
     int rStart = Y0;
     if (YDIR) {
         rStart = Y0 - 2;
-        // the window as it stands after iteration rStart-1 (slot 0 is slid
-        // out before it is read)
+        // rows the first iteration finds in place
 #pragma unroll
-        for (int w = 1; w < WS; ++w) {
-            const int row = rStart - 1 + WLO + w;
-            load_cell<DIM, NPH>(P, P.src, col, row, kz, win[w]);
-            sigwin[w] = useSig ? (T)load_sigma<DIM>(P, col, row, kz) : T(0);
+        for (int m = 2 - R; m < R; ++m) {
+            Cell<DIM, NPH, C> c;
+            loadCell(cm, rStart + m, c);
+            const T sg = sigAt(col, rStart + m);
+            if (m <= 0) {
+                putRow(c, sg, rStart + m, lane + E);
+            } else {
+                win[m] = c;
+                sigwin[m] = sg;
+            }
         }
     }
     // raw values of the row entering the window next iteration
     constexpr bool PF = MarchTuning<T>::kPrefetchRow;
     constexpr bool PU = MarchTuning<T>::kPreloadUpdate && MODE == MODE_FULL;
-    RawCell<DIM, NPH, T> nextRow;
-    if (YDIR && PF) loadRaw(col, rStart + R, nextRow);
+    // the halo column's cell of row r, loaded at the top of the iteration (2D
+    // single phase: 780 -> 765 us per 4096^2 launch; in 3D it costs the third
+    // wave per SIMD, 154 -> 161 us per launch of the two passes at 193x130x97)
+    constexpr bool HPF = YDIR && E > 0 && NPH == 0 && MODE == MODE_FULL;
+    RawCell<DIM, NPH, T> nextRow, haloRow;
+    if (YDIR && PF) loadRaw(cm, rStart + R, nextRow);
     T preU[DIM + 2 + 2 * NPH], preU0[DIM + 2 + 2 * NPH];
+#pragma unroll
+    for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) preU0[q] = T(0);
     // U of the rows between entering the window and their update (R + 1 rows)
     // kept in LDS, each lane its own column: the update reads the cell's U
     // from there instead of from HBM (the row entered R iterations earlier).
@@ -869,94 +941,118 @@ stage_xy_kernel(StageParams<T> P) {
         for (int q = 0; q < NF; ++q) Ghi[q] = T(0);
         double cy = 0.0, dyr = 1.0;
         Cell<DIM, NPH, C> cur;
-        T sigc = T(0);
         if (YDIR) {
 #pragma unroll
-            for (int w = 0; w < WS - 1; ++w) {
-                win[w] = win[w + 1];
-                sigwin[w] = sigwin[w + 1];
+            for (int m = 0; m < R - 1; ++m) {
+                win[m] = win[m + 1];
+                sigwin[m] = sigwin[m + 1];
             }
             if constexpr (PF) {
-                raw_to_cell<DIM, NPH, T>(P, nextRow, win[WS - 1]);
+                raw_to_cell<DIM, NPH, T>(P, nextRow, win[R - 1]);
                 if constexpr (RING) {
                     const int slot = (r + R) % RN;
 #pragma unroll
                     for (int q = 0; q < NCVR; ++q) sUr[slot][q][lane] = nextRow.U[q];
                 }
-                if (r + 1 < Y1) loadRaw(col, r + 1 + R, nextRow);
+                if (r + 1 < Y1) loadRaw(cm, r + 1 + R, nextRow);
             } else {
-                loadCell(col, r + R, win[WS - 1]);
+                loadCell(cm, r + R, win[R - 1]);
             }
-            sigwin[WS - 1] = useSig ? (T)load_sigma<DIM>(P, col, r + R, kz) : T(0);
-            // y reconstruction of row r+1
+            sigwin[R - 1] = sigAt(col, r + R);
+            if (HPF && r >= Y0 && lane < 2 * E) loadRaw(em, r, haloRow);
+            // y reconstruction of row r+1: rows r+2-R .. r+R, up to row r in LDS
             FaceState<DIM, NPH, T> mY, pY;
-            recon_window<DIM, NPH, R, T>(P, win, sigwin, WST, useSig, eps, weno, mY, pY);
+            {
+                T mn[NV], pl[NV], vv[R][NV];
+#pragma unroll
+                for (int m = 0; m < R; ++m) recon_vars<DIM, NPH, T>(win[m], vv[m]);
+                recon_set<R, T, NV>(
+                    [&](int v, int s) __attribute__((always_inline)) {
+                        const int rel = 2 - R + s;
+                        return rel <= 0 ? (T)sp[(r + rel) & 1][v][lane + E] : vv[rel > 0 ? rel - 1 : 0][v];
+                    },
+                    eps, weno, mn, pl);
+                T sm = T(0), sl = T(0);
+                if (useSig)
+                    recon_set<R, T, 1>(
+                        [&](int, int s) __attribute__((always_inline)) {
+                            const int rel = 2 - R + s;
+                            return rel <= 0 ? (T)sp[(r + rel) & 1][NPV - 1][lane + E] : sigwin[rel > 0 ? rel - 1 : 0];
+                        },
+                        eps, weno, &sm, &sl);
+                face_state<DIM, NPH, T>(P, mn, sm, mY);
+                face_state<DIM, NPH, T>(P, pl, sl, pY);
+            }
             if (r >= Y0 - 1) {
                 T F[NFL];
                 riemann<RS, 1, DIM, NPH, T>(plusPrev, mY, incP, igr, F);
-                // cells of face r+1/2: rows r (slot WROW) and r+1 (slot WROW+1)
-                face_contrib<DIM, NPH, T>(F, win[WROW].rho, win[WROW + 1].rho, win[WROW].ar,
-                                          win[WROW + 1].ar, Ghi);
+                // cells of face r+1/2: rows r (LDS) and r+1
+                C rhoL = C(0), arL[NPH > 0 ? NPH : 1];
+                if constexpr (NPH > 0) {
+                    rhoL = sp[r & 1][0][lane + E];
+#pragma unroll
+                    for (int ph = 0; ph < NPH; ++ph) arL[ph] = sar[ph][lane];
+                }
+                face_contrib<DIM, NPH, T>(F, rhoL, win[0].rho, arL, win[0].ar, Ghi);
             }
             plusPrev = pY;
             if (r < Y0) {
+                // warm-up rows: no x phase, no output
 #pragma unroll
                 for (int q = 0; q < NF; ++q) Glo[q] = Ghi[q];
-                continue;  // warm-up rows: no x phase, no output
+                putRow(win[0], sigwin[0], r + 1, lane + E);
+                if constexpr (NPH > 0) {
+#pragma unroll
+                    for (int ph = 0; ph < NPH; ++ph) sar[ph][lane] = win[0].ar[ph];
+                }
+                continue;
             }
             dyr = g.dyw[r + g.ngy];
-            if (PU && owned) {
-                const size_t pid = cell_index(g, col, r, kz);
+            const RowRef idc{row_base(g, r, kz), (unsigned)(cc + g.ngx)};
+            if (PU) {
 #pragma unroll
-                for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) {
-                    preU[q] = P.src[(size_t)q * P.total + pid];
-                    preU0[q] = P.c2 != 0.0 ? P.u0[(size_t)q * P.total + pid] : T(0);
-                }
+                for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) preU[q] = *field_at(P.src, P.total, q, idc);
+            }
+            if (PU && P.c2 != 0.0) {
+#pragma unroll
+                for (int q = 0; q < DIM + 2 + 2 * NPH; ++q) preU0[q] = *field_at(P.u0, P.total, q, idc);
             }
             cy = P.unifY ? cyU : (dxc * dzk) / ((dxc * dyr) * dzk);
-            cur = win[WROW];
-            sigc = sigwin[WROW];
         } else {
-            load_cell<DIM, NPH>(P, P.src, col, r, kz, cur);
-            if (useSig) sigc = (T)load_sigma<DIM>(P, col, r, kz);
+            loadCell(cm, r, cur);
+            putRow(cur, sigAt(col, r), r, lane + E);
             dyr = g.dyw[0];
         }
 
         // ---------------- x phase on row r ----------------
-        __syncthreads();  // previous iteration's LDS reads are complete
-        {
-            T vv[NV];
-            recon_vars<DIM, NPH, T>(cur, vv);
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sp[v][lane + E] = vv[v];
-            if (useSig) sp[NV][lane + E] = sigc;
-        }
         if (E > 0 && lane < 2 * E) {
             Cell<DIM, NPH, C> ce;
-            loadCell(ecol, r, ce);
-            T vv[NV];
-            recon_vars<DIM, NPH, T>(ce, vv);
-            const int pos = lane < E ? lane : kWave + lane;
-#pragma unroll
-            for (int v = 0; v < NV; ++v) sp[v][pos] = vv[v];
-            if (useSig) sp[NV][pos] = (T)load_sigma<DIM>(P, ecol, r, kz);
+            if constexpr (HPF) raw_to_cell<DIM, NPH, T>(P, haloRow, ce);
+            else loadCell(em, r, ce);
+            putRow(ce, sigAt(ecol, r), r, lane < E ? lane : kWave + lane);
         }
         __syncthreads();
+        if (YDIR) {
+            const C* o = &sp[r & 1][0][lane + E];
+            cur.rho = o[0];
+#pragma unroll
+            for (int d = 0; d < DIM; ++d) cur.u[d] = o[(1 + d) * (kWave + 2 * E)];
+            cur.p = o[(DIM + 1) * (kWave + 2 * E)];
+#pragma unroll
+            for (int ph = 0; ph < NPH; ++ph) {
+                cur.a[ph] = o[(DIM + 2 + ph) * (kWave + 2 * E)];
+                cur.ar[ph] = sar[ph][lane];
+            }
+        }
         FaceState<DIM, NPH, T> mX, pX;
         {
-            T st[S], mn[NV], pl[NV];
-#pragma unroll
-            for (int v = 0; v < NV; ++v) {
-#pragma unroll
-                for (int s = 0; s < S; ++s) st[s] = sp[v][lane + s];
-                Recon<R, T>::run(st, eps, weno, mn[v], pl[v]);
-            }
+            T mn[NV], pl[NV];
+            recon_set<R, T, NV>([&](int v, int s) __attribute__((always_inline)) { return (T)sp[r & 1][v][lane + s]; }, eps,
+                                weno, mn, pl);
             T sm = T(0), sl = T(0);
-            if (useSig) {
-#pragma unroll
-                for (int s = 0; s < S; ++s) st[s] = sp[NV][lane + s];
-                Recon<R, T>::run(st, eps, weno, sm, sl);
-            }
+            if (useSig)
+                recon_set<R, T, 1>([&](int, int s) __attribute__((always_inline)) { return (T)sp[r & 1][NPV - 1][lane + s]; },
+                                   eps, weno, &sm, &sl);
             face_state<DIM, NPH, T>(P, mn, sm, mX);
             face_state<DIM, NPH, T>(P, pl, sl, pX);
         }
@@ -998,11 +1094,11 @@ stage_xy_kernel(StageParams<T> P) {
             T acc[NF];
             accumulate<DIM, NPH, T>(acc, FCl, FCx, (T)cx, true);
             if (YDIR) accumulate<DIM, NPH, T>(acc, Glo, Ghi, (T)cy, false);
-            const size_t id = cell_index(g, col, r, kz);
+            const RowRef id{row_base(g, r, kz), (unsigned)(col + g.ngx)};
             if (MODE == MODE_XY) {
 #pragma unroll
                 for (int q = 0; q < NF; ++q)
-                    if (part_slot_used<DIM, NPH, SEMI>(q)) P.part[(size_t)q * P.total + id] = acc[q];
+                    if (part_slot_used<DIM, NPH, SEMI>(q)) *field_at(P.part, P.total, q, id) = acc[q];
             } else {
                 const double h[3] = {dxc, dyr, dzk};
                 double dc;
@@ -1018,7 +1114,7 @@ stage_xy_kernel(StageParams<T> P) {
                         for (int q = 0; q < NCVR; ++q) uring[q] = sUr[r % RN][q][lane];
                     } else {
 #pragma unroll
-                        for (int q = 0; q < NCVR; ++q) uring[q] = P.src[(size_t)q * P.total + id];
+                        for (int q = 0; q < NCVR; ++q) uring[q] = *field_at(P.src, P.total, q, id);
                     }
                     dc = finish_cell<DIM, NPH, SEMI, T, SRC, C>(P, id, acc, cur, h, dt, P.dtPartial != nullptr, uring);
                 } else {
@@ -1030,6 +1126,12 @@ stage_xy_kernel(StageParams<T> P) {
         if (YDIR) {
 #pragma unroll
             for (int q = 0; q < NF; ++q) Glo[q] = Ghi[q];
+            // row r+1 takes row r-1's place
+            putRow(win[0], sigwin[0], r + 1, lane + E);
+            if constexpr (NPH > 0) {
+#pragma unroll
+                for (int ph = 0; ph < NPH; ++ph) sar[ph][lane] = win[0].ar[ph];
+            }
         }
     }
     if (MODE == MODE_FULL && P.dtPartial) {
@@ -1086,6 +1188,7 @@ stage_z_kernel(StageParams<T> P) {
 #pragma unroll
     for (int q = 0; q < NF; ++q) Hlo[q] = T(0);
     const int rStart = Z0 - 2;
+    const ColMap cm = map_column(g, cc);
     // raw values of the plane entering the window next iteration, and the
     // x+y part of the current cell, are loaded one step ahead of their use
     constexpr bool PF = SIFV_PREFETCH_Z;
@@ -1101,17 +1204,19 @@ stage_z_kernel(StageParams<T> P) {
         const int kk = rStart - 1 + WLO + w;
         if (w == WS - 1) {
             RawCell<DIM, NPH, T> rc;
-            load_raw<DIM, NPH, T>(P, P.src, cc, j, kk, rc);
+            load_row<DIM, NPH, T>(P, P.src, cm, j, kk, rc);
 #pragma unroll
             for (int q = 0; q < NCV; ++q) sU[(kk + RING) % RING][q][lane] = rc.U[q];
             raw_to_cell<DIM, NPH, T>(P, rc, win[w]);
         } else {
-            load_cell<DIM, NPH>(P, P.src, cc, j, kk, win[w]);
+            RawCell<DIM, NPH, T> rc;
+            load_row<DIM, NPH, T>(P, P.src, cm, j, kk, rc);
+            raw_to_cell<DIM, NPH, T>(P, rc, win[w]);
         }
         sigwin[w] = useSig ? (T)load_sigma<DIM>(P, cc, j, kk) : T(0);
     }
     RawCell<DIM, NPH, T> nextRow;
-    if (PF) load_raw<DIM, NPH, T>(P, P.src, cc, j, rStart + R, nextRow);
+    if (PF) load_row<DIM, NPH, T>(P, P.src, cm, j, rStart + R, nextRow);
     for (int r = rStart; r < Z1; ++r) {
 #pragma unroll
         for (int w = 0; w < WS - 1; ++w) {
@@ -1122,21 +1227,21 @@ stage_z_kernel(StageParams<T> P) {
 #pragma unroll
             for (int q = 0; q < NCV; ++q) sU[(r + R + RING) % RING][q][lane] = nextRow.U[q];
             raw_to_cell<DIM, NPH, T>(P, nextRow, win[WS - 1]);
-            if (r + 1 < Z1) load_raw<DIM, NPH, T>(P, P.src, cc, j, r + 1 + R, nextRow);
+            if (r + 1 < Z1) load_row<DIM, NPH, T>(P, P.src, cm, j, r + 1 + R, nextRow);
         } else {
             RawCell<DIM, NPH, T> rc;
-            load_raw<DIM, NPH, T>(P, P.src, cc, j, r + R, rc);
+            load_row<DIM, NPH, T>(P, P.src, cm, j, r + R, rc);
 #pragma unroll
             for (int q = 0; q < NCV; ++q) sU[(r + R + RING) % RING][q][lane] = rc.U[q];
             raw_to_cell<DIM, NPH, T>(P, rc, win[WS - 1]);
         }
         sigwin[WS - 1] = useSig ? (T)load_sigma<DIM>(P, cc, j, r + R) : T(0);
         T accPre[NF];
-        if (PP && r >= Z0 && owned) {
-            const size_t pid = cell_index(g, col, j, r);
+        if (PP && r >= Z0) {
+            const RowRef pid{row_base(g, j, r), (unsigned)(cc + g.ngx)};
 #pragma unroll
             for (int q = 0; q < NF; ++q)
-                accPre[q] = part_slot_used<DIM, NPH, SEMI>(q) ? P.part[(size_t)q * P.total + pid] : T(0);
+                accPre[q] = part_slot_used<DIM, NPH, SEMI>(q) ? *field_at(P.part, P.total, q, pid) : T(0);
         }
         FaceState<DIM, NPH, T> mZ, pZ;
         recon_window<DIM, NPH, R, T>(P, win, sigwin, WST, useSig, eps, weno, mZ, pZ);
@@ -1152,11 +1257,11 @@ stage_z_kernel(StageParams<T> P) {
         if (r >= Z0 && owned) {
             const double dzr = g.dzw[r + g.ngz];
             const double cz = P.unifY ? czU : (dxc * dyj) / ((dxc * dyj) * dzr);
-            const size_t id = cell_index(g, col, j, r);
+            const RowRef id{row_base(g, j, r), (unsigned)(col + g.ngx)};
             T acc[NF];
 #pragma unroll
             for (int q = 0; q < NF; ++q)
-                acc[q] = PP ? accPre[q] : (part_slot_used<DIM, NPH, SEMI>(q) ? P.part[(size_t)q * P.total + id] : T(0));
+                acc[q] = PP ? accPre[q] : (part_slot_used<DIM, NPH, SEMI>(q) ? *field_at(P.part, P.total, q, id) : T(0));
             accumulate<DIM, NPH, T>(acc, Hlo, Hhi, (T)cz, false);
             const double h[3] = {dxc, dyj, dzr};
             T Upre[NCV];
