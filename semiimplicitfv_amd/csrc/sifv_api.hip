@@ -352,6 +352,24 @@ void stage_shape(const sifv_handle* h, int& nstrip, int& nseg, int& rows) {
     nseg = (h->ny + rows - 1) / rows;
 }
 
+// Waves per workgroup of the 2D tile kernel (sifv_tile.hpp) for an explicit
+// stage, or 0 for the marching kernel.  Meshes whose marching waves cannot fill
+// the chip take tiles: a wave's serial chain of 6 rows costs 22 us there, a
+// tile 11 us (128^2 FP64; 128^2 water/air 44 -> 16 us, FP32 21 -> 10 us).  The
+// line is where the tiles' halo rows and barriers cost more than that:
+// 576^2 30.4 against 34.9 us and 640^2 36.8 against 35.4 (FP64), 768^2 28.6
+// against 31.7 and 896^2 37.6 against 36.7 (FP32), 800^2 99 against 102
+// (water/air).  Small tiles (2 rows) while those of 8 rows would leave half
+// the 256 CUs idle: 128^2 10.8 against 12.8 us, 320^2 16.0 against 13.7.
+int stage_tile_waves(const sifv_handle* h, bool fp32) {
+    if (h->dim != 2 || h->rowsOverride > 0 || recon_radius(h->cfg.reconOrder) != 3) return 0;
+    if (fp32 && h->nph) return 0;
+    const long cells = (long)h->nx * h->ny;
+    if (cells > (h->nph ? 640000 : fp32 ? 600000 : 360000)) return 0;
+    const long blocks = (long)((h->nx + kOwn - 1) / kOwn) * ((h->ny + kTileWaves - 3) / (kTileWaves - 2));
+    return blocks < 128 ? kTileSmall : kTileWaves;
+}
+
 void zpass_shape(const sifv_handle* h, int& nstrip, int& nseg, int& rows) {
     nstrip = (h->nx + kWave - 1) / kWave;
     if (h->rowsOverride > 0) {
@@ -541,6 +559,13 @@ int launch_stage_p(sifv_handle* h, const T* srcp, const T* u0p, T* dstp, const d
     P.nseg = nseg;
     P.nstrip = nstrip;
     int nb = nstrip * nseg * (h->dim == 3 ? h->nz : 1);
+    const int tw = semi ? 0 : stage_tile_waves(h, sizeof(T) == 4);
+    if (tw) {
+        k.xy = stage_tile_for<T>(h->riemann, h->nph, stage_lean(h->cfg), tw);
+        P.rows = tw - 2;
+        P.nseg = (h->ny + P.rows - 1) / P.rows;
+        nb = nstrip * P.nseg;
+    }
     // viscous / capillary limits of the new state: their own reduction after
     // the stage, into the partial slots after the fused acoustic minima
     const double viscMu = h->cfg.viscousMu > 0.0 ? h->cfg.viscousMu : 0.0;
@@ -561,7 +586,7 @@ int launch_stage_p(sifv_handle* h, const T* srcp, const T* u0p, T* dstp, const d
         rc = launch_stage_slabs<T>(h, k, P, slabs, wantDt, nbs);
         if (rc) return rc;
     } else {
-        rc = timed_launch(h, reinterpret_cast<const void*>(k.xy), dim3(nb), dim3(kWave), args);
+        rc = timed_launch(h, reinterpret_cast<const void*>(k.xy), dim3(nb), dim3(tw ? kWave * tw : kWave), args);
         if (rc) return rc;
     }
     if (wantDt && h->dim < 3) h->npartialValid = nb;

@@ -30,6 +30,16 @@ StageKernels<double> stage_kernels_3d_semi(int R, int rs, int nph);
 StageKernels<float> stage_kernels_fp32(int dim, int R, int rs, bool lean);
 StageKernels<float> stage_kernels_fp32_mp(int dim, int R, int rs);
 
+// Tile form of a full explicit 2D stage (R = 3): nw waves per workgroup
+// (kTileSmall or kTileWaves); null when there is none.
+constexpr int kTileSmall = 4, kTileWaves = 10;
+template <typename T>
+StageFn<T> stage_tile_for(int rs, int nph, bool lean, int nw);
+template <>
+StageFn<double> stage_tile_for<double>(int rs, int nph, bool lean, int nw);
+template <>
+StageFn<float> stage_tile_for<float>(int rs, int nph, bool lean, int nw);
+
 // IGR: pre-pass (rhs, diagonal, rho) per dimension / phase count, and the
 // wavefront Gauss-Seidel sweep per dimension.
 template <typename T>

@@ -1,0 +1,93 @@
+"""The 2D tile stage kernel (meshes too small to fill the GPU with marching
+waves) against the marching kernel over every form that takes it, and against
+the oracle: sizes at the edges of its tiles (62 columns x 2 or 8 rows, the 2-row
+form below 128 tiles of 8 rows), Riemann solvers, reconstructions, RK orders,
+boundary rules, sources, IGR, one and two phases, FP64 and FP32 bulk.
+
+set_tile(rows) selects the marching kernel.  Bars: both kernels evaluate the
+same expressions and differ by the compiler's fused multiply-adds, a few ulp
+per stage: 1e-13 relative Linf after 3 steps in FP64 (1e-9 for water/air, whose
+pressure cancels 2.6e9 against 1e5), 2e-5 in FP32.  Oracle: the 1e-12 bar of the
+explicit tests."""
+import pytest
+
+from semiimplicitfv_amd import (BoundaryCondition as BC, ExplicitSolver, HLLCSolver, LFSolver, ReconstructionOrder as RO,
+                                RusanovSolver)
+from tests.golden import problems
+from tests.helpers import rel_errs
+
+pytestmark = pytest.mark.gpu
+
+RS = {0: LFSolver, 1: RusanovSolver, 2: HLLCSolver}
+WALLS = [BC.NoSlipWall, BC.SlipWall, BC.Symmetry, BC.Outflow, BC.Outflow, BC.Outflow]
+SMALL = [(5, 4), (61, 3), (62, 8), (63, 9), (125, 17)]
+LARGE = [(130, 700), (1000, 71)]   # tiles of 8 rows
+
+
+def _build(n, kind, per):
+    periods = (1, 1, 0) if per else (0, 0, 0)
+    if kind == "two":
+        return problems.make_two_phase_case(2, n, bcs=WALLS, periods=periods, seed=61, p_jump=False)
+    cfg, mesh, st, eos = problems.make_case(2, n, bcs=WALLS, periods=periods, seed=62, nonuniform=kind == "stretched",
+                                            cfl=0.4, shock=kind != "smooth")
+    if kind == "source":
+        cfg.viscousParams.mu = 1e-3
+        cfg.bodyForceParams.a = [0.1, -0.5, 0.0]
+    if kind == "igr":
+        cfg.useIGR = True
+        cfg.igrParams.IGRIters, cfg.igrParams.IGRWarmStartIters = 2, 3
+    return cfg, mesh, st, eos
+
+
+def _fields(cfg, mesh, st, eos, rs, precision, rows, steps=3):
+    g = ExplicitSolver(mesh, RS[rs](eos), eos, None, cfg, precision=precision)
+    g.set_tile(rows)
+    g.upload(st)
+    t, done = g.advance(cfg, steps, 1e30, 0.0)
+    assert done == steps
+    out = {f: mesh.interior(g.download_field(f)).copy() for f in st.field_ids()}
+    g.close()
+    return t, out
+
+
+CASES = [(n, k, rs, per, "fp64") for n in SMALL for k, rs, per in
+         (("plain", 2, False), ("stretched", 1, False), ("plain", 0, True), ("igr", 0, False), ("source", 2, True),
+          ("two", 2, False)) if k != "two" or n != (61, 3)]  # that water/air state fails in the oracle as well
+CASES += [(n, k, rs, per, "fp64") for n in LARGE for k, rs, per in (("plain", 2, True), ("igr", 0, True), ("two", 0, False))]
+CASES += [(n, "smooth", 2, per, "mixed") for n in SMALL[1:] + LARGE for per in (False, True)]
+
+
+@pytest.mark.parametrize("n,kind,rs,per,precision", CASES)
+def test_tile_matches_march(gpu, n, kind, rs, per, precision):
+    cfg, mesh, st, eos = _build(n, kind, per)
+    ta, a = _fields(cfg, mesh, st, eos, rs, precision, 0)
+    tb, b = _fields(cfg, mesh, st, eos, rs, precision, 8)
+    bar = 2e-5 if precision == "mixed" else 1e-9 if kind == "two" else 1e-13
+    assert abs(ta - tb) <= bar * tb
+    for f in a:
+        if abs(b[f]).max() > 0.0:
+            assert rel_errs(a[f], b[f])[1] <= bar, (f, rel_errs(a[f], b[f]))
+        else:
+            assert abs(a[f]).max() == 0.0
+
+
+@pytest.mark.parametrize("rk,recon", [(1, RO.WENO5), (2, RO.UPWIND5), (3, RO.WENO5)])
+@pytest.mark.parametrize("n", [(62, 8), (63, 17), (130, 400)])
+def test_tile_matches_oracle(gpu, oracle_c, n, rk, recon):
+    cfg, mesh, st, eos = problems.make_case(2, n, bcs=WALLS, recon=recon, rk=rk, seed=63, nonuniform=True,
+                                            cfl=0.2 if rk == 1 else 0.4)
+    g = ExplicitSolver(mesh, HLLCSolver(eos), eos, None, cfg)
+    c = oracle_c.CpuSolver(mesh, cfg, 2, eos, "c")
+    sc = st.copy()
+    g.upload(st)
+    for k in range(3):
+        cfg.step = k
+        g.step_resident(cfg)
+        c.explicit_step(sc, cfg)
+    g.download(st)
+    g.close()
+    for f in st.field_ids():
+        if abs(mesh.interior(sc.field(f))).max() == 0.0:
+            continue
+        l1, li = rel_errs(mesh.interior(st.field(f)), mesh.interior(sc.field(f)))
+        assert l1 <= 1e-12 and li <= 1e-12, (f, l1, li)
