@@ -214,9 +214,10 @@ struct sifv_handle {
     int* igrOrder = nullptr;
     double* igrWrap = nullptr;  // wrap side slots of the sweep: x, y, z parts
     // 2D strip-streaming sweep (used when igrStrips > 0)
-    int igrStrips = 0, igrPeriod = 0;
-    double *igrRec = nullptr, *igrEdge = nullptr;
-    int* igrProg = nullptr;
+    int igrStrips = 0, igrPeriod = 0, igrSlots = 0;
+    double* igrRec = nullptr;
+    unsigned long long* igrEdge = nullptr;
+    unsigned igrTag = 1;        // tag of the next solve's initial edge values
     int* igrFlags = nullptr;   // [ntiles] tile epochs, [ntiles] error flag
     int igrNtx = 0, igrNty = 0, igrTj = 1, igrTiles = 0;
     int igrEpoch = 0;
@@ -1662,25 +1663,36 @@ int setup_igr(sifv_handle* h) {
     if (perCu < 1 || cus < 1) return fail(SIFV_ERR_HIP, "IGR sweep kernel cannot be resident");
     h->igrBlocks = std::min(h->igrTiles, perCu * cus);
     // 2D: one wave per 64-column strip when every strip can be resident and
-    // the rows outnumber a strip's lane skew plus two progress chunks (the
-    // wrapping faces of each axis must match: both wrap or neither)
+    // the rows outnumber a strip's lane skew plus the steps prefetched and in
+    // flight (the wrapping faces of each axis must match: both wrap or neither)
     h->igrStrips = 0;
     const int W = (h->nx + kWave - 1) / kWave;
     const bool wrapPair = (h->sbc[0] == BK_WRAP) == (h->sbc[1] == BK_WRAP) &&
                           (h->sbc[2] == BK_WRAP) == (h->sbc[3] == BK_WRAP);
-    if (h->dim == 2 && h->ny >= 2 * kStripChunk + kWave + kStripChunk + 16 && wrapPair) {
+    if (h->dim == 2 && h->ny >= kStripMinRows && wrapPair) {
         int perCuS = 0;
         HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &perCuS, reinterpret_cast<const void*>(igr_strip_kernels().sweep), 2 * kWave, 0));
+            &perCuS, reinterpret_cast<const void*>(igr_strip_kernels().sweep), kStripWaves * kWave, 0));
         if (W <= perCuS * cus) {
             const bool perX = h->sbc[0] == BK_WRAP;
-            const int gap = perX ? std::max(0, W * (kWave + kStripChunk) + kWave + kStripChunk - h->ny) : 0;
+            const int gap = perX ? std::max(0, W * kWave + kWave + 4 * kStripGroup - h->ny) : 0;
             h->igrStrips = W;
             h->igrPeriod = h->ny + gap;
-            HIPCHK(hipMalloc(&h->igrRec, sizeof(double) * (size_t)W * h->ny * kStripSlot));
-            // edge values [2][W][ny] per side, then a sink for lanes without a value
-            HIPCHK(hipMalloc(&h->igrEdge, sizeof(double) * (4 * (size_t)W * h->ny + kWave)));
-            HIPCHK(hipMalloc(&h->igrProg, sizeof(int) * W));
+            h->igrSlots = h->igrPeriod;
+            if (sizeof(double) * (size_t)W * h->igrSlots * kStripSlot > (size_t)2 << 30 && gap > 0) {
+                // slots for the gap rows too would cost more than 2 GiB: as many
+                // slots as rows, and a period of whole multiples of them
+                h->igrSlots = h->ny;
+                h->igrPeriod = (h->igrPeriod + h->ny - 1) / h->ny * h->ny;
+            }
+            HIPCHK(hipMalloc(&h->igrRec, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
+            HIPCHK(hipMemset(h->igrRec, 0, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
+            // tagged edge values [2][W][ny][2] per side (tag 0: none), then a sink
+            // for lanes without a value
+            const size_t ne = sizeof(unsigned long long) * (8 * (size_t)W * h->ny + kWave);
+            HIPCHK(hipMalloc(&h->igrEdge, ne));
+            HIPCHK(hipMemset(h->igrEdge, 0, ne));
+            h->igrTag = 1;
         }
     }
     return SIFV_OK;
@@ -1734,8 +1746,10 @@ int run_igr(sifv_handle* h, int src, const int* active) {
         PA.alpha = A.alpha;
         PA.rec = h->igrRec;
         PA.edgeL = h->igrEdge;
-        PA.edgeR = h->igrEdge + 2 * (size_t)h->igrStrips * h->ny;
+        PA.edgeR = h->igrEdge + 4 * (size_t)h->igrStrips * h->ny;
+        PA.tag = h->igrTag;
         PA.W = h->igrStrips;
+        PA.ns = h->igrSlots;
         void* pargs2[] = {&PA};
         rc = timed_launch(h, reinterpret_cast<const void*>(K.pack), dim3(elementwise_blocks(h)), dim3(256), pargs2);
         if (rc) return rc;
@@ -1745,22 +1759,23 @@ int run_igr(sifv_handle* h, int src, const int* active) {
         SA.rec = h->igrRec;
         SA.edgeL = PA.edgeL;
         SA.edgeR = PA.edgeR;
-        SA.prog = h->igrProg;
+        SA.tag = h->igrTag;
+        h->igrTag += (unsigned)iters + 1;   // tags of one solve: its own
         SA.err = h->igrFlags + h->igrTiles;
         SA.active = active;
         SA.W = h->igrStrips;
         SA.P = h->igrPeriod;
+        SA.ns = h->igrSlots;
         SA.nsweeps = iters;
         SA.perX = h->sbc[0] == BK_WRAP;
         SA.perY = h->sbc[2] == BK_WRAP;
-        HIPCHK(hipMemsetAsync(h->igrProg, 0, sizeof(int) * h->igrStrips, h->stream));
         void* sargs2[] = {&SA};
-        rc = timed_launch(h, reinterpret_cast<const void*>(K.sweep), dim3(h->igrStrips), dim3(2 * kWave), sargs2);
+        rc = timed_launch(h, reinterpret_cast<const void*>(K.sweep), dim3(h->igrStrips), dim3(kStripWaves * kWave), sargs2);
         if (rc) return rc;
         Grid g = h->grid();
         const double* recc = h->igrRec;
         double* sig = h->sigma;
-        void* uargs[] = {&g, &recc, &sig};
+        void* uargs[] = {&g, &recc, &sig, &h->igrSlots};
         rc = timed_launch(h, reinterpret_cast<const void*>(K.unpack), dim3(elementwise_blocks(h)), dim3(256), uargs);
         if (rc) return rc;
         return fill_dirs(h, f, comp, 1, true);
@@ -2152,7 +2167,6 @@ int sifv_destroy(sifv_handle* h) {
     hipFree(h->igrWrap);
     hipFree(h->igrRec);
     hipFree(h->igrEdge);
-    hipFree(h->igrProg);
     hipFree(h->igrFlags);
     for (int q = 0; q < 6; ++q) hipFree(h->jac[q]);
     hipFree(h->resid);

@@ -376,27 +376,53 @@ __global__ void __launch_bounds__(64) igr_sweep_kernel(IgrSweepArgs A) {
 // Per cell the pack kernel stores the five coefficients of the update
 //     new = c0 + cR*right + cT*top + cB*bottom + cL*left,
 // c0 = rhs/diag, cX = alpha/h^2 / rho_face / diag, and sigma, in a cyclic
-// skew: cell (l, j) of a strip sits in slot (j + l) mod ny, so at any step
-// all lanes read one contiguous slot of 64 x 6 doubles (each lane's six
-// values adjacent: three 16-byte loads per lane and step).  A wave may have
-// 63 vector memory operations outstanding, stores included: two groups of
-// kStripGroup steps are loaded ahead (48 loads) and the edge values a chunk
-// produces are gathered in registers and written once per chunk.  Lane 0's left
-// values and the last lane's right values cross strips through edge arrays
-// (by sweep parity), read per chunk of kStripChunk steps after the strip
-// has polled its neighbours' progress (rows completed by their last lane),
-// which every strip publishes at the end of each chunk.  On a wrapping x
-// axis sweep q of strip 0 needs sweep q-1 of the last strip on the same
-// row, while a strip's last lane trails its lane 0 by 63 rows and each strip
-// trails its left neighbour by up to 64 + kStripChunk steps: the gap between
-// sweeps absorbs that skew (gap = W (64 + C) + 64 + C - ny when positive).
+// skew: cell (l, j) of a strip sits in slot (j + l) mod ns, P a multiple of ns, so
+// at step s every lane reads slot s mod ns whatever row and sweep it is at: one
+// contiguous slot of 64 x 6 doubles (three 16-byte loads per lane).  Lane
+// 0's left values and the last lane's right values cross strips through edge
+// arrays (by sweep parity), handed over per group of kStripGroup steps.  On a
+// wrapping x axis sweep q of strip 0 needs sweep q-1 of the last strip on the same
+// row, while each strip trails its left neighbour by 64 steps and more: the gap
+// between sweeps makes room for that skew (gap = 64 W + 64 + 4 groups - ny when
+// positive, 72 steps more than the dependencies need).
+// What bounds it: the serial chain of a group (8 steps of two dependent multiply-
+// adds and a shift, with the LDS reads and counters around them about 0.65 us)
+// times (ny + 64 W) / 8, and around a wrapping axis the hand-off of every strip
+// (about 8 us beyond the 64 steps).  Microseconds a sweep, one wave with loads,
+// coefficients and sweeps in one and a release / acquire hand-off -> now: 1024^2
+// wrapping 468 -> 251, 1024^2 walls 240 -> 148, 2048^2 981 -> 536 and 580 -> 325.
 // Ghost semantics are those of the per-sweep scalar fill: zero-gradient
 // faces read the cell's own previous-sweep value, wrapping y faces the
 // previous result (bottom) and the saved previous-sweep row-0 value (top).
-constexpr int kStripGroup = 8;     // steps per prefetch group
-constexpr int kStripBufs = 3;      // groups held in registers: two in flight while one is used
-constexpr int kStripChunk = kStripGroup * kStripBufs;   // steps per progress hand-off
-constexpr int kStripSlot = 6 * kWave;   // doubles per record slot: [lane][c0, cL, cR, cB, cT, sigma]
+constexpr int kStripGroup = 8;     // steps per group: of loads, of computation, of hand-off
+constexpr int kStripMinRows = 152; // lane skew, prefetched steps and a margin: a sweep's records are written before they are read again
+// A record slot (doubles): three arrays of 64 pairs, (c0, cR), (cT, sigma
+// of the cell in the next slot, that is of the row above), (cB, cL), so each of a
+// step's three 16-byte loads per lane is one contiguous KB (with the six values of
+// a lane adjacent every load touched all 24 lines of the slot), and a step needs
+// nothing of the next one's records (with a cell's own sigma in its slot the +y
+// operand of a group's last step waited for the next group, halving the distance
+// of the loads ahead); the cell's own old value is the step before's +y operand.
+constexpr int kStripSlot = 6 * kWave;
+__device__ __forceinline__ size_t strip_sigma(int lane) { return 2 * kWave + 2 * (size_t)lane + 1; }
+
+// An edge value handed from strip to strip: two 64-bit words, each half of the
+// value beside the tag of the sweep it belongs to, stored and loaded at device
+// scope (past the XCDs' L2s).  A reader polls the words themselves: no fence, which
+// would write back or invalidate an L2 shared by other strips, and no progress
+// flag, whose store has to wait for the values' and whose poll is one more round
+// trip (1024^2 wrapping: 330 us a sweep, with fences and flags 356).
+__device__ __forceinline__ void edge_store(unsigned long long* p, double v, unsigned tag) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v), t = (unsigned long long)tag << 32;
+    __hip_atomic_store(p, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool edge_load(const unsigned long long* p, unsigned tag, double& v) {
+    const unsigned long long a = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long b = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __longlong_as_double((long long)((b << 32) | (a & 0xffffffffull)));
+    return (unsigned)(a >> 32) == tag && (unsigned)(b >> 32) == tag;
+}
 
 struct IgrStripPackArgs {
     Grid g;
@@ -405,10 +431,12 @@ struct IgrStripPackArgs {
     const double* rhs;
     const double* diag;
     double alpha;
-    double* rec;           // [W][ny][6][64]
-    double* edgeL;         // [2][W][ny]
-    double* edgeR;         // [2][W][ny]
+    double* rec;           // [W][ns] record slots
+    unsigned long long* edgeL;   // [2][W][ny][2]
+    unsigned long long* edgeR;   // [2][W][ny][2]
+    unsigned tag;          // of the initial iterate's edge values
     int W;
+    int ns;                // slots per strip
 };
 
 // Threads run in record order (strip, slot, lane): each wave writes one
@@ -418,336 +446,455 @@ template <int DIM>
 __global__ void __launch_bounds__(256) igr_strip_pack_kernel(IgrStripPackArgs A) {
     const Grid& g = A.g;
     const size_t sy = (size_t)g.nxT;
-    const size_t total = (size_t)A.W * g.ny * kWave;
+    const size_t total = (size_t)A.W * A.ns * kWave;
     for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
         const int l = (int)(e % kWave);
         const size_t ws = e / kWave;
-        const int t = (int)(ws % g.ny), w = (int)(ws / g.ny);
+        const int t = (int)(ws % A.ns), w = (int)(ws / A.ns);
         const int i = w * kWave + l;
         if (i >= g.nx) continue;
         int j = t - l;
-        if (j < 0) j += g.ny;
+        if (j < 0) j += A.ns;
+        double2* r = reinterpret_cast<double2*>(A.rec + ws * kStripSlot) + l;
+        if (j >= g.ny) {
+            // the gap slot before row 0 holds row 0's sigma
+            if (j == A.ns - 1) r[kWave].y = A.sigma[cell_index(g, i, 0, 0)];
+            continue;
+        }
         const size_t id = cell_index(g, i, j, 0);
         const double ri = A.rho[id];
         const double rd = 1.0 / A.diag[id];
         const double hx = g.dxw[i + g.ngx], hy = g.dyw[j + g.ngy];
         const double ax = A.alpha / (hx * hx), ay = A.alpha / (hy * hy);
-        double2* r = reinterpret_cast<double2*>(A.rec + ws * kStripSlot + 6 * l);
         const double sg = A.sigma[id];
-        r[0] = make_double2(A.rhs[id] * rd, ax / (0.5 * (ri + A.rho[id - 1])) * rd);
-        r[1] = make_double2(ax / (0.5 * (ri + A.rho[id + 1])) * rd, ay / (0.5 * (ri + A.rho[id - sy])) * rd);
-        r[2] = make_double2(ay / (0.5 * (ri + A.rho[id + sy])) * rd, sg);
+        // the row above; above the last row only when the slots wrap there
+        const double up = A.sigma[cell_index(g, i, j + 1 < g.ny ? j + 1 : 0, 0)];
+        r[0] = make_double2(A.rhs[id] * rd, ax / (0.5 * (ri + A.rho[id + 1])) * rd);
+        r[kWave] = make_double2(ay / (0.5 * (ri + A.rho[id + sy])) * rd, up);
+        r[2 * kWave] = make_double2(ay / (0.5 * (ri + A.rho[id - sy])) * rd, ax / (0.5 * (ri + A.rho[id - 1])) * rd);
         // edge values of "sweep -1" (parity slot 1): the initial iterate
         const int L = min(kWave - 1, g.nx - 1 - w * kWave);
-        if (l == 0) A.edgeL[((size_t)A.W + w) * g.ny + j] = sg;
-        if (l == L) A.edgeR[((size_t)A.W + w) * g.ny + j] = sg;
+        if (l == 0) edge_store(A.edgeL + 2 * (((size_t)A.W + w) * g.ny + j), sg, A.tag);
+        if (l == L) edge_store(A.edgeR + 2 * (((size_t)A.W + w) * g.ny + j), sg, A.tag);
     }
 }
 
 template <int DIM>
-__global__ void __launch_bounds__(256) igr_strip_unpack_kernel(Grid g, const double* rec, double* sigma) {
+__global__ void __launch_bounds__(256) igr_strip_unpack_kernel(Grid g, const double* rec, double* sigma, int ns) {
     int i, j, k;
     for (InteriorIter it_(g.nx, g.ny, 1); it_.next(i, j, k);) {
         const int w = i / kWave, l = i - w * kWave;
-        int t = j + l;
-        if (t >= g.ny) t -= g.ny;
-        sigma[cell_index(g, i, j, 0)] = rec[((size_t)w * g.ny + t) * kStripSlot + 6 * l + 5];
+        int t = j + l - 1;
+        t = t < 0 ? t + ns : t >= ns ? t - ns : t;
+        sigma[cell_index(g, i, j, 0)] = rec[((size_t)w * ns + t) * kStripSlot + strip_sigma(l)];
     }
 }
 
 struct IgrStripArgs {
     int nx, ny;
     double* rec;
-    double* edgeL;
-    double* edgeR;
-    int* prog;             // [W] schedule rows completed by the strip's last lane; zero at launch
+    unsigned long long* edgeL;
+    unsigned long long* edgeR;
+    unsigned tag;          // of the initial iterate's edge values; sweep q's carry tag + q + 1
     int* err;
     const int* active;
     int W, P, nsweeps;
+    int ns;                // record slots per strip; P is a multiple of it
     int perX, perY;
 };
 
-__device__ __forceinline__ double dpp_shr1(double v) {   // lane l <- lane l-1
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x138, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x138, 0xF, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
 __device__ __forceinline__ double dpp_shl1(double v) {   // lane l <- lane l+1
     const long long b = __double_as_longlong(v);
     const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x130, 0xF, 0xF, true);
     const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x130, 0xF, 0xF, true);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-__device__ __forceinline__ double read_lane(double v, int k) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)b, k);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+// The same shifts with the lane that has no source (0 / 63) taking edge's value.
+__device__ __forceinline__ double dpp_shr1_in(double v, double edge) {
+    const long long b = __double_as_longlong(v), e = __double_as_longlong(edge);
+    const int lo = __builtin_amdgcn_update_dpp((int)e, (int)b, 0x138, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(b >> 32), 0x138, 0xF, 0xF, false);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-
-// Largest schedule row in [a, b] that is a real row (not a gap row, inside
-// the launch's [0, Rt)), or -1.
-__device__ __forceinline__ int strip_last_row(int a, int b, int P, int ny, int Rt) {
-    b = min(b, Rt - 1);
-    if (b < a || b < 0) return -1;
-    const int jb = b % P;
-    const int r = jb < ny ? b : b - jb + ny - 1;
-    return r >= a && r >= 0 ? r : -1;
+__device__ __forceinline__ double dpp_shl1_in(double v, double edge) {
+    const long long b = __double_as_longlong(v), e = __double_as_longlong(edge);
+    const int lo = __builtin_amdgcn_update_dpp((int)e, (int)b, 0x130, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(b >> 32), 0x130, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
-
-// Two waves per strip.  Wave 0 computes; wave 1 carries the strip's traffic
-// with its neighbours through LDS: it publishes each chunk wave 0 finishes
-// (edge values to the edge arrays, release, progress flag) and loads the
-// neighbours' edge values of upcoming chunks as soon as their progress
-// allows (acquire), up to kStripRing chunks ahead.  Wave 0 thus never waits
-// on a device-scope fence, which would drain its prefetch pipeline.  Wave 1
-// never blocks on one duty: each pass of its loop publishes what it can and
-// loads what it can.  Neither wave branches on its lane index at a loop
-// boundary (stores of lanes without a value go to a sink element).
-constexpr int kStripRing = 8;
+// Seven waves per strip, one duty each, so that the serial chain holds nothing
+// that does not depend on it and the duties' round trips do not add up:
+//   wave 0 carries the sweeps: new = base + cB*bottom + cL*left;
+//   waves 1 and 2 bring the records (even and odd groups), two groups each in
+//     registers on their way from memory and up to kStripRecGroups in LDS;
+//   wave 3 works out base = c0 + cR*right + cT*top, which has previous-sweep
+//     values only, in place of c0 in the LDS record;
+//   wave 4 publishes the edge values of the groups wave 0 finishes;
+//   waves 5 and 6 poll the left and the right neighbour's edge values of upcoming
+//     groups, up to kStripRing steps ahead.
+// A record is loaded again no earlier than P - 8 (kStripRecGroups + 4) steps after
+// the step that stored its sigma; wave 0 has at most seven groups of stores
+// outstanding when it counts a group as done, so that store is complete for every
+// P >= 129 (waiting for all but two groups made the stores' latency the limit).
+// Every wait is bounded and ends on the abort flag.
+constexpr int kStripRecGroups = 5;
+constexpr int kStripWaves = 7;
+constexpr int kStripRing = 192;   // steps of wave 0's results and inputs held in LDS
 
 template <int DIM>
-__global__ void __launch_bounds__(128) igr_strip_kernel(IgrStripArgs A) {
+__global__ void __launch_bounds__(64 * kStripWaves) igr_strip_kernel(IgrStripArgs A) {
     if (A.active && *A.active == 0) return;
-    constexpr int U = kStripGroup, C = kStripChunk, NR = kStripRing;
-    __shared__ double sIn[NR][2][kWave];    // neighbours' values for wave 0: [slot][left/right][chunk step]
-    __shared__ double sOut[NR][C][kWave];   // wave 0's results: [slot][chunk step][lane]
-    __shared__ int sFlag[4];                // chunks done by wave 0, loaded for it, published; abort
+    constexpr int U = kStripGroup, RS = kStripRing, RG = kStripRecGroups;
+    static_assert(RS % U == 0 && RS >= 2 * kWave, "whole groups; helpers move up to a wave of steps at once");
+    __shared__ __align__(16) double sIn[2][RS];  // neighbours' values: [left/right][step mod RS]
+    __shared__ double sOut[RS][2];               // wave 0's results of lanes 0 and L: [step mod RS]
+    __shared__ double2 sRec[RG * U][3][kWave];   // records: [step mod RG U]
+    // groups: [0] left inputs loaded, [1] right inputs loaded, [2] published,
+    // [3] abort, [4] done by wave 0, [5], [6] even / odd record groups loaded,
+    // [7] bases worked out
+    __shared__ int sFlag[8];
     const int w = blockIdx.x, lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);   // wave-uniform
-    const int ny = A.ny, P = A.P, W = A.W;
+    const int ny = A.ny, P = A.P, W = A.W, ns = A.ns;
     const int L = min(kWave - 1, A.nx - 1 - w * kWave);
     const int Rt = A.nsweeps * P;
     const int nsteps = Rt + kWave - 1;
-    const int nchunks = (nsteps + C - 1) / C;
+    const int ngroups = (nsteps + U - 1) / U;
     const bool leftWall = w == 0 && !A.perX, rightWall = w == W - 1 && !A.perX;
     const int leftSrc = w > 0 ? w - 1 : W - 1, rightSrc = w < W - 1 ? w + 1 : 0;
-    if (threadIdx.x < 4) sFlag[threadIdx.x] = 0;
+    double* rec = A.rec + (size_t)w * ns * kStripSlot;
+    if (threadIdx.x < 8) sFlag[threadIdx.x] = 0;
     __syncthreads();
     auto lds_load = [](int* p) __attribute__((always_inline)) { return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP); };
     auto lds_store = [](int* p, int v) __attribute__((always_inline)) { __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP); };
-    // wave 1 watches the device error flag and raises the block's abort flag,
-    // which wave 0 polls in LDS (a device-scope load would make wave 0 wait
-    // for its whole prefetch pipeline)
+    // the helper waves watch the device error flag and raise the block's abort
+    // flag, which waves 0 and 3 poll in LDS
     auto aborted = [&]() __attribute__((always_inline)) { return __hip_atomic_load(&sFlag[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0; };
-    if (wave == 1) {
-        double* sink = A.edgeL + 4 * (size_t)W * ny;
-        int nextPub = 0, nextIn = 0, knownL = 0, knownR = 0, idle = 0;
-        while (nextPub < nchunks) {
-            bool moved = false;
-            // publish every chunk wave 0 has finished: edge values, then one
-            // release and the progress of the last of them
-            const int aDone = lds_load(&sFlag[0]);
-            if (aDone > nextPub) {
-                for (int c = nextPub; c < aDone; ++c) {
-                    const int s0 = c * C, slot = c % NR;
-                    int r = s0 + lane;
-                    bool v = lane < C && r < Rt && r % P < ny;
-                    double* dl = v ? A.edgeL + ((size_t)((r / P) & 1) * W + w) * ny + r % P : sink;
-                    r = s0 + lane - L;
-                    v = lane < C && r >= 0 && r < Rt && r % P < ny;
-                    double* dr = v ? A.edgeR + ((size_t)((r / P) & 1) * W + w) * ny + r % P : sink;
-                    *dl = sOut[slot][min(lane, C - 1)][0];
-                    *dr = sOut[slot][min(lane, C - 1)][L];
-                }
-                const int done = min(max(min(aDone * C, nsteps) - L, 0), Rt);
-                __threadfence();
-                __hip_atomic_store(&A.prog[w], done, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                lds_store(&sFlag[2], aDone);
-                nextPub = aDone;
-                moved = true;
+    // one idle pass of a helper wave; true: give up
+    auto idle_pass = [&](int& idle) __attribute__((always_inline)) {
+        const bool budget = ++idle > (1 << 25);
+        if (budget) __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (aborted() || ((idle & 255) == 0 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+            __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            return true;
+        }
+        return budget;
+    };
+    if (wave == 4) {
+        int pub = 0, idle = 0;
+        while (pub < ngroups) {
+            const int done = min(lds_load(&sFlag[4]), pub + kWave / U);
+            if (done == pub) {
+                if (idle_pass(idle)) return;
+                continue;
             }
-            // load the inputs of every chunk whose slot is free and whose rows
-            // the neighbours have published: one acquire for all of them
-            const int upto = min(nchunks, aDone + NR);
-            if (nextIn < upto) {
-                int nlL = knownL, nlR = knownR;
-                auto need = [&](int c, int& nL, int& nR) __attribute__((always_inline)) {
-                    const int s0 = c * C;
-                    nL = 0;
-                    nR = 0;
-                    if (!leftWall) {
-                        const int r = strip_last_row(s0, s0 + C - 1, P, ny, Rt);
-                        if (r >= 0) nL = w > 0 ? r + 1 : r - P + 1;
-                    }
-                    if (!rightWall) {
-                        const int r = strip_last_row(s0 - L, s0 + C - 1 - L, P, ny, Rt);
-                        if (r >= 0) nR = r - P + 1;
-                    }
-                };
-                int nL, nR;
-                need(nextIn, nL, nR);
-                if (nL > nlL) nlL = __hip_atomic_load(&A.prog[leftSrc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (nR > nlR) nlR = __hip_atomic_load(&A.prog[rightSrc], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                knownL = nlL;
-                knownR = nlR;
-                int last = nextIn;
-                while (last < upto) {
-                    need(last, nL, nR);
-                    if (nL > knownL || nR > knownR) break;
-                    ++last;
+            idle = 0;
+            const int s = pub * U + lane;
+            const bool in = s < done * U;
+            const double* o = sOut[s % RS];
+            int r = s;
+            bool v = in && r < Rt && r % P < ny;
+            if (v) edge_store(A.edgeL + 2 * (((size_t)((r / P) & 1) * W + w) * ny + r % P), o[0], A.tag + r / P + 1);
+            r = s - L;
+            v = in && r >= 0 && r < Rt && r % P < ny;
+            if (v)
+                edge_store(A.edgeR + 2 * (((size_t)((r / P) & 1) * W + w) * ny + r % P), o[L > 0 ? 1 : 0],
+                           A.tag + r / P + 1);
+            lds_store(&sFlag[2], done);
+            pub = done;
+        }
+        return;
+    }
+    if (wave == 1 || wave == 2) {
+        const int odd = wave - 1;
+        double ra[6][U], rb[6][U];
+        int tp = odd * U % ns;   // slot of the next step loaded
+        auto load = [&](double (&r)[6][U]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const double2* p = reinterpret_cast<const double2*>(rec + (size_t)tp * kStripSlot) + lane;
+#pragma unroll
+                for (int f = 0; f < 3; ++f) {
+                    const double2 v = p[f * kWave];
+                    r[2 * f][k] = v.x;
+                    r[2 * f + 1][k] = v.y;
                 }
-                if (last > nextIn) {
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                    for (int c = nextIn; c < last; ++c) {
-                        const int s0 = c * C, slot = c % NR;
-                        int r = s0 + lane;
-                        bool v = lane < C && !leftWall && r < Rt && r % P < ny;
-                        int q = v ? r / P : 0, j = v ? r % P : 0;
-                        const double a = A.edgeR[v ? ((size_t)((w > 0 ? q : q - 1) & 1) * W + leftSrc) * ny + j : 0];
-                        r = s0 + lane - L;
-                        const bool vr = lane < C && !rightWall && r >= 0 && r < Rt && r % P < ny;
-                        q = vr ? r / P : 0;
-                        j = vr ? r % P : 0;
-                        const double b = A.edgeL[vr ? ((size_t)((q - 1) & 1) * W + rightSrc) * ny + j : 0];
-                        sIn[slot][0][lane] = v ? a : 0.0;
-                        sIn[slot][1][lane] = vr ? b : 0.0;
-                    }
-                    lds_store(&sFlag[1], last);
-                    nextIn = last;
-                    moved = true;
-                }
+                if (++tp == ns) tp = 0;
             }
-            if (moved) {
-                idle = 0;
+            tp = (tp + U) % ns;
+        };
+        int idle = 0;
+        auto put = [&](int g, const double (&r)[6][U]) __attribute__((always_inline)) {
+            while (lds_load(&sFlag[4]) + RG <= g)
+                if (idle_pass(idle)) return false;
+            idle = 0;
+#pragma unroll
+            for (int k = 0; k < U; ++k)
+#pragma unroll
+                for (int f = 0; f < 3; ++f)
+                    sRec[g % RG * U + k][f][lane] = make_double2(r[2 * f][k], r[2 * f + 1][k]);
+            lds_store(&sFlag[5 + odd], g + 1);
+            return true;
+        };
+        load(ra);
+        load(rb);
+        for (int g = odd; g < ngroups; g += 4) {
+            if (!put(g, ra)) return;
+            load(ra);
+            if (g + 2 >= ngroups) return;
+            if (!put(g + 2, rb)) return;
+            load(rb);
+        }
+        return;
+    }
+    if (wave >= 5) {
+        const bool right = wave == 6;
+        int* loadedFlag = &sFlag[right ? 1 : 0];
+        if (right ? rightWall : leftWall) {
+            lds_store(loadedFlag, ngroups);
+            return;
+        }
+        const int src = right ? rightSrc : leftSrc;
+        const unsigned long long* edges = right ? A.edgeL : A.edgeR;
+        const int back = !right && w > 0 ? 0 : 1;   // sweeps back
+        int loaded = 0, idle = 0;
+        int span = 1;   // groups polled at once: one while waiting, so that the polls leave the memory to others
+        while (loaded < ngroups) {
+            // slots of groups wave 0 has finished are free again
+            const int upto = min(min(ngroups, lds_load(&sFlag[4]) + RS / U), loaded + span);
+            // lane m polls the value of step loaded U + m: the row of lane 0 (left)
+            // or of the last lane (right)
+            const int s = loaded * U + lane;
+            const int r = s - (right ? L : 0);
+            const bool v = s < upto * U && r >= 0 && r < Rt && r % P < ny;
+            double a = 0.0;
+            bool ready = s < upto * U;
+            if (v) {
+                const int q = r / P - back;
+                ready = edge_load(edges + 2 * (((size_t)(q & 1) * W + src) * ny + r % P), A.tag + q + 1, a);
+            }
+            // groups whose every step is there, from the front
+            const unsigned long long ok = __ballot(ready);
+            const int got = (ok == ~0ull ? kWave : __builtin_ctzll(~ok)) / U;
+            if (got == 0) {
+                span = 1;
+                if (idle_pass(idle)) return;
+                continue;
+            }
+            span = min(2 * span, kWave / U);
+            idle = 0;
+            if (lane < got * U) sIn[right ? 1 : 0][s % RS] = a;
+            loaded += got;
+            lds_store(loadedFlag, loaded);
+        }
+        return;
+    }
+    // waves 0 and 3 read their counters together and ahead of need; see() is where
+    // they are looked at, and orders what is read after it
+    auto peek = [&](int f) __attribute__((always_inline)) { return __hip_atomic_load(&sFlag[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    auto see = [&]() __attribute__((always_inline)) { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup"); };
+    const double* sig0 = rec + strip_sigma(lane);
+    // (cell (lane, j)'s sigma is in slot j + lane - 1)
+    const double first = sig0[(size_t)(lane > 0 ? lane - 1 : ns - 1) * kStripSlot];   // row 0 of the initial iterate
+    if (wave == 3) {
+        // row 0 of the previous sweep; +y operand of the step before (the cell's own
+        // old value); row in the period of the lane's next step
+        double row0 = first, above = sig0[(size_t)(ns - 1) * kStripSlot];
+        int jc = lane == 0 ? 0 : P - lane;
+        // the period's row of lane 63 at the group's first step, slot of the group
+        int pos = P - (kWave - 1), r0 = 0, i0 = 0;
+        int inR = 0, recs[2] = {0, 0}, idle = 0;
+        auto bases = [&](int g, int odd) __attribute__((always_inline)) {
+            while (recs[odd] <= g || inR <= g) {
+                const int e = peek(5), o = peek(6), n = peek(1), ab = peek(3);
+                recs[0] = __builtin_amdgcn_readfirstlane(e);
+                recs[1] = __builtin_amdgcn_readfirstlane(o);
+                inR = __builtin_amdgcn_readfirstlane(n);
+                if (recs[odd] > g && inR > g) break;
+                if (__builtin_amdgcn_readfirstlane(ab) != 0 || idle_pass(idle)) return false;
+            }
+            see();
+            idle = 0;
+            double2 cr[U], ct[U];
+            double rv[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                rv[k] = sIn[1][i0 + k];
+                cr[k] = sRec[r0 + k][0][lane];
+                ct[k] = sRec[r0 + k][1][lane];
+            }
+            if (leftWall && lane == 0) {
+                // beyond the wall: the cell's own old value
+#pragma unroll
+                for (int k = 0; k < U; ++k) sIn[0][i0 + k] = k > 0 ? ct[k > 0 ? k - 1 : 0].y : above;
+            }
+            if (pos >= 1 && pos + kWave + U - 2 <= ny - 2 && L == kWave - 1) {
+                // every lane at an interior row, and the neighbour's value comes in at
+                // the lane without a source of the shift
+                if (rightWall) {
+#pragma unroll
+                    for (int k = 0; k < U; ++k) rv[k] = k > 0 ? ct[k > 0 ? k - 1 : 0].y : above;
+                }
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    const double right = dpp_shl1_in(ct[k].y, rv[k]);
+                    sRec[r0 + k][0][lane].x = cr[k].x + cr[k].y * right + ct[k].x * ct[k].y;
+                }
+                above = ct[U - 1].y;
+                jc += U;
             } else {
-                const bool budget = ++idle > (1 << 25);
-                if (budget) __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (budget || __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || aborted()) {
-                    __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    return;
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    const double sgT = ct[k].y, cellOld = above;
+                    above = sgT;
+                    const double top = jc < ny - 1 ? sgT : (A.perY ? row0 : cellOld);
+                    const double rightS = dpp_shl1(sgT);
+                    const double right = lane < L ? rightS : (rightWall ? cellOld : rv[k]);
+                    sRec[r0 + k][0][lane].x = cr[k].x + cr[k].y * right + ct[k].x * top;
+                    // at a period's end the slot holds the sweep's own row 0
+                    if (++jc == P) {
+                        row0 = sgT;
+                        jc = 0;
+                    }
                 }
-                __builtin_amdgcn_s_sleep(1);
             }
+            lds_store(&sFlag[7], g + 1);
+            if ((pos += U) >= P) pos -= P;
+            if ((r0 += U) == RG * U) r0 = 0;
+            if ((i0 += U) == RS) i0 = 0;
+            return true;
+        };
+        for (int g = 0; g < ngroups; g += 2) {
+            if (!bases(g, 0)) return;
+            if (g + 1 < ngroups && !bases(g + 1, 1)) return;
         }
         return;
     }
     // wave 0: the sweeps
+    __builtin_amdgcn_s_setprio(3);
     const bool act = lane <= L;
-    double* rec = A.rec + (size_t)w * ny * kStripSlot + 6 * lane;
-    // lane state: row 0 of the current and of the previous sweep, last result
-    double row0 = rec[(size_t)lane * kStripSlot + 5];           // slot of (lane, 0) = lane
-    int tl = ny - 1 + lane;
-    if (tl >= ny) tl -= ny;
-    double last = A.perY ? rec[(size_t)tl * kStripSlot + 5] : row0;
-    double row0old = row0;
-    // schedule position of the lane at the next compute step and at the
-    // next prefetch step: row in the period and sweep
+    double* sig = rec + strip_sigma(lane);
+    // lane state: row 0 of the previous sweep, last result
+    double row0 = first;
+    int tl = ny - 2 + lane;
+    if (tl >= ns) tl -= ns;
+    double last = A.perY ? sig[(size_t)tl * kStripSlot] : row0;
+    // row in the period of the lane's next step, and of lane 63's at the group's
+    // first; slot the next step's result goes to; places of the group in the rings
     int jc = lane == 0 ? 0 : P - lane;
-    int jp = jc;
-    double buf[kStripBufs][6][U];
-    auto prefetch = [&](double (&bf)[6][U]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int k = 0; k < U; ++k) {
-            int t = jp < ny ? jp + lane : lane;
-            if (t >= ny) t -= ny;
-            const double2* r = reinterpret_cast<const double2*>(rec + (size_t)t * kStripSlot);
-#pragma unroll
-            for (int f = 0; f < 3; ++f) {
-                const double2 v = r[f];
-                bf[2 * f][k] = v.x;
-                bf[2 * f + 1][k] = v.y;
-            }
-            if (++jp == P) jp = 0;
-        }
+    int pos = P - (kWave - 1), tc = ns - 1, r1 = 0, i0 = 0;
+    // the lanes whose results the neighbours read
+    const bool edge = lane == 0 || lane == L;
+    const int edgeCol = lane == 0 ? 0 : 1;
+    double base[2][U];
+    double2 cbl[2][U];
+    // left inputs and bases of a group there, and its output slots published by wave
+    // 4: the counters last seen
+    int inL = 0, pub = 0, done3 = 0, spins = 0;
+    auto count = [&](int l, int d, int p) __attribute__((always_inline)) {
+        inL = __builtin_amdgcn_readfirstlane(l);
+        done3 = __builtin_amdgcn_readfirstlane(d);
+        pub = __builtin_amdgcn_readfirstlane(p);
     };
-    // lane k holds lane 0's left value and the last lane's right value of
-    // chunk step k (read once per chunk from LDS, picked per step by readlane:
-    // an LDS read per step would wait behind the previous step's LDS write)
-    double lchunk = 0.0, rchunk = 0.0;
-    // a group in which every lane's row is an interior row (1 .. ny-2) of one
-    // sweep: all lanes update, none meets a boundary row, and all lanes write
-    // the same record slot (s - qP mod ny); lanes past the mesh edge write
-    // their padding records
-    auto group = [&](int g0, int s0, int slot, const double (&cur)[6][U], const double (&nxt)[6][U]) __attribute__((always_inline)) {
-        const int lo = g0 - (kWave - 1), hi = g0 + U - 1;
-        const int q = lo >= 0 ? lo / P : -1;
-        if (lo >= 0 && hi < Rt && lo - q * P >= 1 && hi - q * P <= ny - 2) {
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                const int kk = g0 + k - s0;
-                const double sgT = k < U - 1 ? cur[5][k + 1] : nxt[5][0];
-                const double cellOld = cur[5][k];
-                const double rightS = dpp_shl1(sgT);
-                const double leftS = dpp_shr1(last);
-                const double lv = read_lane(lchunk, kk), rv = read_lane(rchunk, kk);
-                const double right = lane < L ? rightS : (rightWall ? cellOld : rv);
-                const double left = lane > 0 ? leftS : (leftWall ? cellOld : lv);
-                const double base = cur[0][k] + cur[2][k] * right + cur[4][k] * sgT;
-                const double nw = base + cur[3][k] * last + cur[1][k] * left;
-                int t = g0 + k - q * P;
-                if (t >= ny) t -= ny;
-                rec[(size_t)t * kStripSlot + 5] = nw;
-                sOut[slot][kk][lane] = nw;
-                last = nw;
-            }
-            jc += U;
-        } else {
-            // general steps: any row position (first or last row of a sweep,
-            // gap rows, rows outside the launch)
-#pragma unroll
-            for (int k = 0; k < U; ++k) {
-                const int s = g0 + k, kk = s - s0;
-                if (s >= nsteps) break;
-                const double sgT = k < U - 1 ? cur[5][k + 1] : nxt[5][0];
-                const int r = s - lane;
-                const bool valid = act && r >= 0 && r < Rt && jc < ny;
-                const double sendR = jc + 1 == P ? row0 : sgT;
-                const double rightS = dpp_shl1(sendR);
-                const double leftS = dpp_shr1(last);
-                const double cellOld = cur[5][k];
-                const double top = jc < ny - 1 ? sgT : (A.perY ? row0old : cellOld);
-                const double bot = jc > 0 || A.perY ? last : row0;
-                const double lv = read_lane(lchunk, kk), rv = read_lane(rchunk, kk);
-                const double right = lane < L ? rightS : (rightWall ? cellOld : rv);
-                const double left = lane > 0 ? leftS : (leftWall ? cellOld : lv);
-                const double base = cur[0][k] + cur[2][k] * right + cur[4][k] * top;
-                const double nw = base + cur[3][k] * bot + cur[1][k] * left;
-                if (valid) {
-                    if (jc == 0) {
-                        row0old = row0;
-                        row0 = nw;
-                    }
-                    int t = jc + lane;
-                    if (t >= ny) t -= ny;
-                    rec[(size_t)t * kStripSlot + 5] = nw;
-                    last = nw;
-                }
-                sOut[slot][kk][lane] = nw;
-                if (++jc == P) jc = 0;
-            }
-        }
-    };
-    auto wait_flag = [&](int* f, int v) __attribute__((always_inline)) {
-        int spins = 0;
-        while (lds_load(f) < v) {
-            if (aborted()) return false;
+    auto wait = [&](int g, int gBase) __attribute__((always_inline)) {
+        while (inL <= g || done3 <= gBase || pub <= g - RS / U) {
+            const int l = peek(0), d = peek(7), p = peek(2), ab = peek(3);
+            count(l, d, p);
+            if (__builtin_amdgcn_readfirstlane(ab) != 0) return false;
             if (++spins > (1 << 27)) {
                 __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 return false;
             }
-            __builtin_amdgcn_s_sleep(1);
         }
+        see();
+        spins = 0;
         return true;
     };
-    prefetch(buf[0]);
-    prefetch(buf[1]);
-    for (int c = 0; c < nchunks; ++c) {
-        const int s0 = c * C, slot = c % NR;
-        // inputs of the chunk loaded, and the output slot published by wave 1
-        if (!wait_flag(&sFlag[1], c + 1)) return;
-        if (!wait_flag(&sFlag[2], c + 1 - NR)) return;
-        lchunk = sIn[slot][0][lane];
-        rchunk = sIn[slot][1][lane];
-        prefetch(buf[2]);
-        group(s0, s0, slot, buf[0], buf[1]);
-        prefetch(buf[0]);
-        group(s0 + U, s0, slot, buf[1], buf[2]);
-        prefetch(buf[1]);
-        group(s0 + 2 * U, s0, slot, buf[2], buf[0]);
-        lds_store(&sFlag[0], c + 1);
+    // next group's records (after the last group: of any old one, unused)
+    auto fetch = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < U; ++k) {
+            base[b][k] = sRec[r1 + k][0][lane].x;
+            cbl[b][k] = sRec[r1 + k][2][lane];
+        }
+        if ((r1 += U) == RG * U) r1 = 0;
+    };
+    // byte offsets of the lane's sigma in the slots of a group
+    unsigned sigOff[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) sigOff[k] = 8 * (unsigned)(k * kStripSlot + strip_sigma(lane));
+    auto group = [&](int g, int b) __attribute__((always_inline)) {
+        double (*out)[2] = &sOut[i0];
+        // the neighbour's values, the same in every lane; read before the next
+        // group's records, behind which they would wait
+        double lv[U];
+        int l, d, p;
+        auto read = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < U; ++k) lv[k] = sIn[0][i0 + k];
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(1 - b);
+            l = peek(0), d = peek(7), p = peek(2);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (pos >= 1 && pos + kWave + U - 2 <= ny - 2 && tc + U <= ns) {
+            // every lane's row is an interior row (1 .. ny-2) of one sweep: all lanes
+            // update, none meets a boundary row, and all write the same record slot
+            // (lanes past the mesh edge their padding records)
+            read();
+            char* dst = reinterpret_cast<char*>(rec + (size_t)tc * kStripSlot);
+            double nw[U];
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const double left = dpp_shr1_in(last, lv[k]);
+                last = nw[k] = base[b][k] + cbl[b][k].x * last + cbl[b][k].y * left;
+                *reinterpret_cast<double*>(dst + sigOff[k]) = last;
+            }
+            if (edge) {
+#pragma unroll
+                for (int k = 0; k < U; ++k) out[k][edgeCol] = nw[k];
+            }
+            jc += U;
+            if ((tc += U) == ns) tc = 0;
+        } else {
+            // general steps: any row position (first or last row of a sweep,
+            // gap rows, rows outside the launch)
+            read();
+#pragma unroll
+            for (int k = 0; k < U; ++k) {
+                const int s = g * U + k;
+                if (s >= nsteps) break;
+                const int r = s - lane;
+                const bool valid = act && r >= 0 && r < Rt && jc < ny;
+                const double bot = jc > 0 || A.perY ? last : row0;
+                const double left = dpp_shr1_in(last, lv[k]);
+                const double nw = base[b][k] + cbl[b][k].x * bot + cbl[b][k].y * left;
+                if (valid) {
+                    if (jc == 0) row0 = nw;
+                    sig[(size_t)tc * kStripSlot] = nw;
+                    last = nw;
+                }
+                if (edge) out[k][edgeCol] = nw;
+                if (++jc == P) jc = 0;
+                if (++tc == ns) tc = 0;
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(56)" ::: "memory");   // stores of all but seven groups are done
+        lds_store(&sFlag[4], g + 1);
+        count(l, d, p);
+        if ((pos += U) >= P) pos -= P;
+        if ((i0 += U) == RS) i0 = 0;
+    };
+    if (!wait(-1, 0)) return;
+    fetch(0);
+    for (int g = 0; g < ngroups; g += 2) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            if (g + b >= ngroups) return;
+            if (!wait(g + b, min(g + b + 1, ngroups - 1))) return;
+            group(g + b, b);
+        }
     }
 }
 

@@ -57,7 +57,7 @@ IgrSweepFn igr_sweep_kernel_for(int dim);
 struct IgrStripKernels {
     void (*pack)(IgrStripPackArgs);
     void (*sweep)(IgrStripArgs);
-    void (*unpack)(Grid, const double*, double*);
+    void (*unpack)(Grid, const double*, double*, int);
 };
 IgrStripKernels igr_strip_kernels();
 
