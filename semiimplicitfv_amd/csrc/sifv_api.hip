@@ -977,11 +977,18 @@ dim3 semi_brick_grid(const sifv_handle* h) {
                 (h->nz + kSemiBrickPlanes - 1) / kSemiBrickPlanes);
 }
 
-// Grid of the tiled sweeps (jacobi_tile_kernel): 64-column x kTileRows-row tiles,
-// kTilePlanes planes per block in 3D.
+// Grid of the tiled sweeps (jacobi_tile_kernel): 64-column x 4-row tiles, kTilePlanes
+// planes per block in 3D.
 dim3 jacobi_tile_grid(const sifv_handle* h) {
-    return dim3((h->nx + 63) / 64, (h->ny + kTileRows - 1) / kTileRows,
+    const int rows = kTileThreads / kWave;
+    return dim3((h->nx + kWave - 1) / kWave, (h->ny + rows - 1) / rows,
                 h->dim >= 3 ? (h->nz + kTilePlanes - 1) / kTilePlanes : 1);
+}
+
+template <typename T, int MODE>
+const void* jacobi_tile_fn(const sifv_handle* h) {
+    return h->dim == 2 ? reinterpret_cast<const void*>(jacobi_tile_kernel<T, MODE, 1>)
+                       : reinterpret_cast<const void*>(jacobi_tile_kernel<T, MODE, kTileDepth>);
 }
 
 int run_jacobi(sifv_handle* h, const double* rho, const double* dt, double tol, int maxIter, int* n) {
@@ -1025,8 +1032,8 @@ int run_jacobi(sifv_handle* h, const double* rho, const double* dt, double tol, 
                     Jt.pin = h->jac[k % 2];
                     Jt.pout = h->jac[(k + 1) % 2];
                     void* cargs[] = {&Jt};
-                    e = hipLaunchKernel(reinterpret_cast<const void*>(jacobi_tile_kernel<double, TILE_SWEEP64>),
-                                        jacobi_tile_grid(h), dim3(64, kTileRows), cargs, 0, h->stream);
+                    e = hipLaunchKernel(jacobi_tile_fn<double, TILE_SWEEP64>(h),
+                                        jacobi_tile_grid(h), dim3(kTileThreads), cargs, 0, h->stream);
                 }
                 hipGraph_t gr = nullptr;
                 const hipError_t ec = hipStreamEndCapture(h->stream, &gr);
@@ -1046,8 +1053,8 @@ int run_jacobi(sifv_handle* h, const double* rho, const double* dt, double tol, 
                 Jt.pin = h->jac[it % 2];
                 Jt.pout = h->jac[(it + 1) % 2];
                 void* args[] = {&Jt};
-                rc = timed_launch(h, reinterpret_cast<const void*>(jacobi_tile_kernel<double, TILE_SWEEP64>), jacobi_tile_grid(h),
-                                  dim3(64, kTileRows), args);
+                rc = timed_launch(h, jacobi_tile_fn<double, TILE_SWEEP64>(h), jacobi_tile_grid(h),
+                                  dim3(kTileThreads), args);
             } else {
                 J.iter = it;
                 J.pin = h->jac[it % 2];
@@ -1165,8 +1172,8 @@ int run_jacobi_mixed(sifv_handle* h, const double* rho, const double* dt, double
             Mt.pout = pout;
             Mt.iter = slot;
             void* args[] = {&Mt};
-            rc = timed_launch(h, reinterpret_cast<const void*>(jacobi_tile_kernel<double, TILE_PASS>),
-                              jacobi_tile_grid(h), dim3(64, kTileRows), args);
+            rc = timed_launch(h, jacobi_tile_fn<double, TILE_PASS>(h),
+                              jacobi_tile_grid(h), dim3(kTileThreads), args);
         } else {
             M.pin = pin;
             M.din = din;
@@ -1192,8 +1199,8 @@ int run_jacobi_mixed(sifv_handle* h, const double* rho, const double* dt, double
                 St.pin = d;
                 St.pout = dbuf[q % 2];
                 void* sargs[] = {&St};
-                rc = timed_launch(h, reinterpret_cast<const void*>(jacobi_tile_kernel<float, TILE_SWEEP32>), jacobi_tile_grid(h),
-                                  dim3(64, kTileRows), sargs);
+                rc = timed_launch(h, jacobi_tile_fn<float, TILE_SWEEP32>(h), jacobi_tile_grid(h),
+                                  dim3(kTileThreads), sargs);
             } else {
                 S.din = d;
                 S.dout = dbuf[q % 2];
@@ -1687,9 +1694,8 @@ int setup_igr(sifv_handle* h) {
             }
             HIPCHK(hipMalloc(&h->igrRec, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
             HIPCHK(hipMemset(h->igrRec, 0, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
-            // tagged edge values [2][W][ny][2] per side (tag 0: none), then a sink
-            // for lanes without a value
-            const size_t ne = sizeof(unsigned long long) * (8 * (size_t)W * h->ny + kWave);
+            // tagged edge values [2][W][ny][2] per side (tag 0: none)
+            const size_t ne = sizeof(unsigned long long) * 8 * (size_t)W * h->ny;
             HIPCHK(hipMalloc(&h->igrEdge, ne));
             HIPCHK(hipMemset(h->igrEdge, 0, ne));
             h->igrTag = 1;

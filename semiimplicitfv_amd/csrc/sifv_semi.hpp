@@ -442,23 +442,28 @@ __global__ void __launch_bounds__(256) jacobi32_kernel(Jacobi32Args A) {
 
 // ---- Tiled Jacobi sweeps (2D/3D) ----------------------------------------------------
 // The Jacobi kernels above (the FP64 update with its max-norm, the FP32 correction
-// sweep and the FP64 pass of the mixed solve) organised for HBM: a block of
-// 64 x kTileRows threads owns a tile of 64 columns x kTileRows rows and marches it
-// through up to kTilePlanes planes of z.  The z-neighbours of p and rho stay in
-// registers; each plane's p and rho tile with a one-cell x/y halo is staged in LDS,
-// double-buffered by plane parity (one barrier per plane).  Lanes on the halo
-// column i == nx / row j == ny load it; the tile's outer halo comes from extra
-// loads by lanes 0 / 63 and rows 0 / kTileRows-1.  p goes through the scalar ghost
-// rule, rho through its filled ghosts.  Per cell the arithmetic is the elementwise
-// kernels' expression for expression, so both forms give identical bits.
-#ifndef SIFV_JACOBI_TILE_ROWS
-#define SIFV_JACOBI_TILE_ROWS 4
-#endif
+// sweep and the FP64 pass of the mixed solve): a block of 256 threads owns a tile of
+// 64 columns x 4 rows and marches it through up to kTilePlanes planes of z.  The
+// z-neighbours of p and rho stay in registers; each plane's (p, rho) pairs with a
+// one-cell x/y halo, which the block's first 2 (64 + 4) threads load, are staged in
+// LDS, double-buffered by plane parity (one barrier per plane).  In 3D the operands
+// of the next kTileDepth planes are in flight.  p goes through the scalar ghost rule,
+// rho through its filled ghosts.
+// What bounds it: the memory's latency and 40 B a cell.  At 160 x 144 x 176: seven
+// IEEE divisions a cell, a branch per load and the operands loaded in the plane that
+// needs them 49 us a sweep (420 instructions a cell and plane, 13 us of them issue
+// now); one reciprocal (1 / (a b) times b and a) for the two faces of a direction,
+// loads one plane ahead 47; four planes ahead 44 (two 44, eight-plane tiles 49,
+// 32-plane 46, tiles of 32 x 8 the same).  Five such arrays stream in 25.
 #ifndef SIFV_JACOBI_TILE_PLANES
 #define SIFV_JACOBI_TILE_PLANES 16
 #endif
-constexpr int kTileRows = SIFV_JACOBI_TILE_ROWS;
 constexpr int kTilePlanes = SIFV_JACOBI_TILE_PLANES;
+constexpr int kTileThreads = 256;
+#ifndef SIFV_JACOBI_DEPTH
+#define SIFV_JACOBI_DEPTH 4
+#endif
+constexpr int kTileDepth = SIFV_JACOBI_DEPTH;   // planes in flight in 3D
 
 enum TileMode : int { TILE_SWEEP64 = 0, TILE_SWEEP32 = 1, TILE_PASS = 2 };
 
@@ -482,27 +487,54 @@ struct JacobiTileArgs {
     float* co32;         // dt^2 rho c^2 in FP32
 };
 
-template <typename T>
-__device__ __forceinline__ T tile_coef(T r, T dL, T hc) {
-    if constexpr (sizeof(T) == 8) return 1.0 / (dmax_ref(r, 1e-14) * dL * hc);
-    else return __builtin_amdgcn_rcpf(fmaxf(r, 1e-14f) * dL * hc);
+// The two face coefficients 1 / (max(rho_face, 1e-14) dist h) of a direction from
+// the sums of the cell's and the neighbours' densities; dl, dr: half the face
+// distances times the cell's width.  FP64 callers pass sums of at least 2e-14 (or
+// clamp them): a NaN stays one.
+__device__ __forceinline__ void face_pair(double sl, double sr, double dl, double dr, double& cl, double& cr) {
+    const double a = sl * dl, b = sr * dr;
+    const double r = rcp_nr(a * b);
+    cl = b * r;
+    cr = a * r;
+}
+__device__ __forceinline__ void face_pair(float sl, float sr, float dl, float dr, float& cl, float& cr) {
+    cl = __builtin_amdgcn_rcpf(fmaxf(sl, 2e-14f) * dl);
+    cr = __builtin_amdgcn_rcpf(fmaxf(sr, 2e-14f) * dr);
 }
 
-template <typename T, int MODE>
-__global__ void __launch_bounds__(64 * kTileRows) jacobi_tile_kernel(JacobiTileArgs<T> A) {
+// A copy in a register of its own.  (A plain one shares v's register, so that the load
+// that refills v goes elsewhere and is waited for at the loop's end to be copied back.)
+__device__ __forceinline__ double moved(double v) {
+    double o;
+    asm("v_mov_b64 %0, %1" : "=v"(o) : "v"(v));
+    return o;
+}
+__device__ __forceinline__ float moved(float v) {
+    float o;
+    asm("v_mov_b32 %0, %1" : "=v"(o) : "v"(v));
+    return o;
+}
+
+template <typename T>
+struct alignas(2 * sizeof(T)) TilePair {
+    T p, r;
+};
+
+template <typename T, int MODE, int D>
+__global__ void __launch_bounds__(kTileThreads) jacobi_tile_kernel(JacobiTileArgs<T> A) {
     constexpr bool F64 = sizeof(T) == 8;
     constexpr bool PASS = MODE == TILE_PASS;
     static_assert(F64 == (MODE != TILE_SWEEP32), "FP64 sweeps and passes, FP32 sweeps");
-    constexpr int TY = kTileRows;
+    constexpr int W = kWave, TY = kTileThreads / W;
     if constexpr (MODE == TILE_SWEEP64) {
         // converged at an earlier iteration: nothing left to do
         if (A.iter > 0 && A.resid[A.iter - 1] < A.tol) return;
     }
-    __shared__ T sp[2][TY + 2][66];
-    __shared__ T sr[2][TY + 2][66];
-    __shared__ double sh[TY];
+    __shared__ TilePair<T> st[2][TY + 2][W + 2];
+    __shared__ double sh[kTileThreads / kWave];
+    __shared__ T sdz[kTilePlanes][2];   // (half face distances times width) of z: a load in the loop would wait for the ones in flight
     const Grid& g = A.g;
-    const bool z = A.dim >= 3;
+    constexpr bool z = D > 1;   // a 2D mesh is one plane
     // launch order deals blocks round-robin to the 8 XCDs: hand each XCD a
     // contiguous run of tiles so that neighbouring tiles share its L2
     int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
@@ -516,164 +548,193 @@ __global__ void __launch_bounds__(64 * kTileRows) jacobi_tile_kernel(JacobiTileA
             bz = t / (gx * gy);
         }
     }
-    const int tx = threadIdx.x, ty = threadIdx.y;
-    const int i0 = bx * 64, j0 = by * TY;
-    const int i = i0 + tx, j = j0 + ty;
+    const int tid = threadIdx.x, tx = tid % W, ty = tid / W;
+    const int i0 = bx * W, j0 = by * TY;
+    const int wv = min(W, g.nx - i0), hv = min(TY, g.ny - j0);   // cells of a ragged tile
+    const bool active = tx < wv && ty < hv;
+    // lanes past the mesh read its last cell and store nothing
+    const int i = i0 + min(tx, wv - 1), j = j0 + min(ty, hv - 1);
     const int k0 = z ? bz * kTilePlanes : 0, k1 = z ? min(g.nz, k0 + kTilePlanes) : 1;
-    const long sy = g.nxT, sz = (long)g.nxT * g.nyT;
-    auto raw = [&](int a, int b, int c) {
-        return (long)(a + g.ngx) + sy * (long)(b + g.ngy) + sz * (long)(c + g.ngz);
-    };
-    const bool active = i < g.nx && j < g.ny;
-    const bool loads = i <= g.nx && j <= g.ny;
-    const int ic = min(i, g.nx), jc = min(j, g.ny);
-    const long pofs = (long)(map_axis_scalar(ic, g.nx, g.sbc[0], g.sbc[1]) - ic) +
-                      (long)(map_axis_scalar(jc, g.ny, g.sbc[2], g.sbc[3]) - jc) * sy;
-    const bool xh = (tx == 0 || (tx == 63 && i0 + 64 <= g.nx)) && j < g.ny;
-    const bool yh = (ty == 0 || (ty == TY - 1 && j0 + TY <= g.ny)) && i < g.nx;
-    const int hi = tx == 0 ? i0 - 1 : i0 + 64, hj = ty == 0 ? j0 - 1 : j0 + TY;
-    const int xs = tx == 0 ? 0 : 65, ys = ty == 0 ? 0 : TY + 1;
-    const long hx = raw(hi, jc, k0), hy = raw(ic, hj, k0);
-    const long hxP = (long)(map_axis_scalar(hi, g.nx, g.sbc[0], g.sbc[1]) - hi);
-    const long hyP = (long)(map_axis_scalar(hj, g.ny, g.sbc[2], g.sbc[3]) - hj) * sy;
+    const size_t sz = (size_t)g.nxT * g.nyT;
+    const unsigned own = (unsigned)((j - j0) * g.nxT + (i - i0));   // from the tile's first cell
+    const size_t org = (size_t)(i0 + g.ngx) + (size_t)g.nxT * (j0 + g.ngy);
+    // this thread's halo cell: (gi, gj), its rho there and its p at the mapped cell
+    int gi = i, gj = j;
+    bool halo;
+    if (tid < 2 * TY) {
+        halo = (tid >> 1) < hv;
+        gi = tid & 1 ? i0 + wv : i0 - 1;
+        gj = j0 + (tid >> 1);
+    } else {
+        const int e = tid - 2 * TY;
+        halo = e < 2 * W && e % W < wv;
+        gi = i0 + e % W;
+        gj = e < W ? j0 - 1 : j0 + hv;
+    }
+    // (threads without one read the tile's first cell: no branch among the loads)
+    size_t hr = org, hp = org;
+    TilePair<T>* hs = &st[0][0][0];
+    if (halo) {
+        hr = (size_t)(gi + g.ngx) + (size_t)g.nxT * (gj + g.ngy);
+        hp = (size_t)(map_axis_scalar(gi, g.nx, g.sbc[0], g.sbc[1]) + g.ngx) +
+             (size_t)g.nxT * (map_axis_scalar(gj, g.ny, g.sbc[2], g.sbc[3]) + g.ngy);
+        hs = &st[0][gj - j0 + 1][gi - i0 + 1];
+    }
+    constexpr int SB = (TY + 2) * (W + 2);   // pairs of one buffer
     const bool hasP = A.pin != nullptr;
     const bool hasD = PASS && A.din != nullptr;
     // p of the sweep: the iterate; of the pass: iterate + FP32 correction
-    auto ldp = [&](long q) -> T {
-        if constexpr (PASS) return hasD ? A.pin[q] + (double)A.din[q] : A.pin[q];
-        else return A.pin[q];
+    auto ldp = [&](size_t base, size_t q) __attribute__((always_inline)) -> T {
+        if constexpr (PASS) return hasD ? (A.pin + base)[q] + (double)(A.din + base)[q] : (A.pin + base)[q];
+        else if constexpr (F64) return (A.pin + base)[q];
+        else return hasP ? (A.pin + base)[q] : T(0);
     };
-    auto zofs = [&](int k) { return (long)(map_axis_scalar(k, g.nz, g.sbc[4], g.sbc[5]) - k) * sz; };
-    T hcx = 0, dLx = 0, dRx = 0, hcy = 0, dLy = 0, dRy = 0;
-    if (active) {
-        const T hlx = (T)g.dxw[i - 1 + g.ngx], hrx = (T)g.dxw[i + 1 + g.ngx];
-        hcx = (T)g.dxw[i + g.ngx];
-        dLx = T(0.5) * (hlx + hcx);
-        dRx = T(0.5) * (hcx + hrx);
-        const T hly = (T)g.dyw[j - 1 + g.ngy], hry = (T)g.dyw[j + 1 + g.ngy];
-        hcy = (T)g.dyw[j + g.ngy];
-        dLy = T(0.5) * (hly + hcy);
-        dRy = T(0.5) * (hcy + hry);
-    }
+    auto plane = [&](int k) __attribute__((always_inline)) { return sz * (size_t)(k + g.ngz); };
+    const int zlo = map_axis_scalar(-1, g.nz, g.sbc[4], g.sbc[5]), zhi = map_axis_scalar(g.nz, g.nz, g.sbc[4], g.sbc[5]);
+    auto planeP = [&](int k) __attribute__((always_inline)) { return plane(k < 0 ? zlo : k >= g.nz ? zhi : k); };
+    // half face distances times the cell's width
+    const T hx = (T)g.dxw[i + g.ngx], hy = (T)g.dyw[j + g.ngy];
+    const T dLx = T(0.5) * (T(0.5) * ((T)g.dxw[i - 1 + g.ngx] + hx)) * hx;
+    const T dRx = T(0.5) * (T(0.5) * (hx + (T)g.dxw[i + 1 + g.ngx])) * hx;
+    const T dLy = T(0.5) * (T(0.5) * ((T)g.dyw[j - 1 + g.ngy] + hy)) * hy;
+    const T dRy = T(0.5) * (T(0.5) * (hy + (T)g.dyw[j + 1 + g.ngy])) * hy;
     double dt2 = 0.0;
     if constexpr (F64) {
         const double dt = *A.dt;
         dt2 = dt * dt;
     }
-    long id = raw(ic, jc, k0);
-    T pzm = 0, pc = 0, pzp = 0, rzm = 0, rc = 0, rzp = 0;
-    T hpx = 0, hrx = 0, hpy = 0, hry = 0;
-    if (loads) {
-        rc = A.rho[id];
-        if (hasP) pc = ldp(id + pofs);
-        if (z) {
-            rzm = A.rho[id - sz];
-            if (hasP) pzm = ldp(id + pofs - sz + zofs(k0 - 1));
-        }
+    if (z && tid < k1 - k0) {
+        const int c = k0 + tid + g.ngz;
+        const T hl = (T)g.dzw[c - 1], hc = (T)g.dzw[c], hr2 = (T)g.dzw[c + 1];
+        sdz[tid][0] = T(0.5) * (T(0.5) * (hl + hc)) * hc;
+        sdz[tid][1] = T(0.5) * (T(0.5) * (hc + hr2)) * hc;
     }
-    if (xh) {
-        hrx = A.rho[hx];
-        if (hasP) hpx = ldp(hx + hxP);
+    // in flight: own p and rho of the planes from k + 2, the halo's and the other
+    // operands of the planes from k; the last planes' loads are repeated
+    T fp[D], fr[D], hpv[D], hrv[D], fc[D], fs[D];
+    auto load_own = [&](int s, int k) __attribute__((always_inline)) {
+        const int c = min(k, k1);
+        fp[s] = ldp(planeP(c) + org, own);
+        fr[s] = (A.rho + plane(c) + org)[own];
+    };
+    auto load_plane = [&](int s, int k) __attribute__((always_inline)) {
+        const size_t pl = plane(min(k, k1 - 1));
+        hpv[s] = ldp(pl, hp);
+        hrv[s] = (A.rho + pl)[hr];
+        fc[s] = (A.co + pl + org)[own];
+        fs[s] = (A.rhs + pl + org)[own];
+    };
+    T pzm = 0, pzp = 0, rzm = 0, rzp = 0;
+    T pc = ldp(plane(k0) + org, own), rc = (A.rho + plane(k0) + org)[own];
+    if (z) {
+        pzm = ldp(planeP(k0 - 1) + org, own);
+        rzm = (A.rho + plane(k0 - 1) + org)[own];
+        pzp = ldp(planeP(k0 + 1) + org, own);
+        rzp = (A.rho + plane(k0 + 1) + org)[own];
     }
-    if (yh) {
-        hry = A.rho[hy];
-        if (hasP) hpy = ldp(hy + hyP);
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+        load_plane(s, k0 + s);
+        if (D > 1) load_own(s, k0 + 2 + s);
     }
     double mr = 0.0;
-    for (int k = k0; k < k1; ++k) {
+    auto step = [&](int k, int s) __attribute__((always_inline)) {
         const int b = k & 1;
-        sp[b][ty + 1][tx + 1] = pc;
-        sr[b][ty + 1][tx + 1] = rc;
-        if (xh) {
-            sp[b][ty + 1][xs] = hpx;
-            sr[b][ty + 1][xs] = hrx;
-        }
-        if (yh) {
-            sp[b][ys][tx + 1] = hpy;
-            sr[b][ys][tx + 1] = hry;
-        }
-        // operands of this plane not staged in LDS, and the next plane's halo
-        if (loads && z) {
-            rzp = A.rho[id + sz];
-            if (hasP) pzp = ldp(id + pofs + sz + zofs(k + 1));
-        }
-        T q2 = 0, qs = 0;
-        if (active) {
-            q2 = A.co[id];
-            qs = A.rhs[id];
-        }
-        const long dk = (long)(k + 1 - k0) * sz;
-        T nhpx = 0, nhrx = 0, nhpy = 0, nhry = 0;
-        if (k + 1 < k1) {
-            if (xh) {
-                nhrx = A.rho[hx + dk];
-                if (hasP) nhpx = ldp(hx + dk + hxP);
-            }
-            if (yh) {
-                nhry = A.rho[hy + dk];
-                if (hasP) nhpy = ldp(hy + dk + hyP);
-            }
-        }
+        if (active) st[b][ty + 1][tx + 1] = {pc, rc};
+        if (halo) hs[b * SB] = {hpv[s], hrv[s]};
+        const T q2 = fc[s], qs = fs[s];
+        if (D > 1) load_plane(s, k + D);
         __syncthreads();
-        if (active) {
-            T off = 0, diag = 0;
-            {
-                const T rL = T(0.5) * (rc + sr[b][ty + 1][tx]), rR = T(0.5) * (rc + sr[b][ty + 1][tx + 2]);
-                const T cL = tile_coef(rL, dLx, hcx), cR = tile_coef(rR, dRx, hcx);
-                off += cL * sp[b][ty + 1][tx] + cR * sp[b][ty + 1][tx + 2];
-                diag += cL + cR;
-            }
-            {
-                const T rL = T(0.5) * (rc + sr[b][ty][tx + 1]), rR = T(0.5) * (rc + sr[b][ty + 2][tx + 1]);
-                const T cL = tile_coef(rL, dLy, hcy), cR = tile_coef(rR, dRy, hcy);
-                off += cL * sp[b][ty][tx + 1] + cR * sp[b][ty + 2][tx + 1];
-                diag += cL + cR;
-            }
+        {
+            const TilePair<T>* c = &st[b][ty + 1][tx + 1];
+            const TilePair<T> xl = c[-1], xr = c[1], yl = c[-(W + 2)], yr = c[W + 2];
+            T sxl = rc + xl.r, sxr = rc + xr.r, syl = rc + yl.r, syr = rc + yr.r, szl = 0, szr = 0;
+            T dlz = 0, drz = 0;
             if (z) {
-                const T hl = (T)g.dzw[k - 1 + g.ngz], hc = (T)g.dzw[k + g.ngz], hr = (T)g.dzw[k + 1 + g.ngz];
-                const T rL = T(0.5) * (rc + rzm), rR = T(0.5) * (rc + rzp);
-                const T cL = tile_coef(rL, T(0.5) * (hl + hc), hc), cR = tile_coef(rR, T(0.5) * (hc + hr), hc);
+                dlz = sdz[k - k0][0];
+                drz = sdz[k - k0][1];
+                szl = rc + rzm;
+                szr = rc + rzp;
+            }
+            if constexpr (F64) {
+                // densities under the floor are rare: look once for all faces (a NaN
+                // is under nothing, and stays)
+                double lo = fmin(fmin(sxl, sxr), fmin(syl, syr));
+                if (z) lo = fmin(lo, fmin(szl, szr));
+                if (__builtin_expect(lo < 2e-14, 0)) {
+                    sxl = dmax_ref(sxl, 2e-14);
+                    sxr = dmax_ref(sxr, 2e-14);
+                    syl = dmax_ref(syl, 2e-14);
+                    syr = dmax_ref(syr, 2e-14);
+                    szl = dmax_ref(szl, 2e-14);
+                    szr = dmax_ref(szr, 2e-14);
+                }
+            }
+            T cL, cR;
+            face_pair(sxl, sxr, dLx, dRx, cL, cR);
+            T off = cL * xl.p + cR * xr.p, diag = cL + cR;
+            face_pair(syl, syr, dLy, dRy, cL, cR);
+            off += cL * yl.p + cR * yr.p;
+            diag += cL + cR;
+            if (z) {
+                face_pair(szl, szr, dlz, drz, cL, cR);
                 off += cL * pzm + cR * pzp;
                 diag += cL + cR;
             }
-            if constexpr (PASS) {
+            const size_t id = plane(k) + org;
+            if constexpr (F64) {
                 const double co = q2 * dt2;
                 const double den = 1.0 + co * diag;
-                const double pn = (qs + co * off) / den;
-                A.pout[id] = pc;
-                A.pn[id] = pn;
-                A.r32[id] = (float)(den * (pn - pc));
-                A.co32[id] = (float)co;
-                mr = dmax_ref(mr, fabs(pn - pc));
-            } else if constexpr (F64) {
-                const double co = q2 * dt2;
-                const double den = 1.0 + co * diag;
-                const double pn = (qs + co * off) / den;
-                A.pout[id] = pn;
-                mr = dmax_ref(mr, fabs(pn - pc));
-            } else {
-                A.pout[id] = (qs + q2 * off) * __builtin_amdgcn_rcpf(1.0f + q2 * diag);
+                const double pn = div_fast(qs + co * off, den);
+                const double up = fabs(pn - pc);
+                if (active) {
+                    mr = dmax_ref(mr, up);
+                    if constexpr (PASS) {
+                        (A.pout + id)[own] = pc;
+                        (A.pn + id)[own] = pn;
+                        (A.r32 + id)[own] = (float)(den * (pn - pc));
+                        (A.co32 + id)[own] = (float)co;
+                    } else {
+                        (A.pout + id)[own] = pn;
+                    }
+                }
+            } else if (active) {
+                (A.pout + id)[own] = (qs + q2 * off) * __builtin_amdgcn_rcpf(1.0f + q2 * diag);
             }
         }
         pzm = pc;
         pc = pzp;
         rzm = rc;
         rc = rzp;
-        hpx = nhpx;
-        hrx = nhrx;
-        hpy = nhpy;
-        hry = nhry;
-        id += sz;
+        if (D > 1) {
+            pzp = moved(fp[s]);
+            rzp = moved(fr[s]);
+            __builtin_amdgcn_sched_barrier(0);
+            load_own(s, k + 2 + D);
+        }
+    };
+    // whole groups without a branch between the steps, which would make each wait
+    // for the loads it has just issued
+    int k = k0;
+    for (; k + D <= k1; k += D) {
+#pragma unroll
+        for (int s = 0; s < D; ++s) step(k + s, s);
     }
+#pragma unroll
+    for (int s = 0; s + 1 < D; ++s)
+        if (k + s < k1) step(k + s, s);
     if constexpr (F64) {
         const double w = wave_max(mr);
-        if (tx == 0) sh[ty] = w;
+        if (tid % kWave == 0) sh[tid / kWave] = w;
         __syncthreads();
-        if (tx == 0 && ty == 0) {
+        if (tid == 0) {
             double m = 0.0;
-            for (int q = 0; q < TY; ++q) m = dmax_ref(m, sh[q]);
-            atomicMax(reinterpret_cast<unsigned long long*>(&A.resid[A.iter]),
-                      (unsigned long long)__double_as_longlong(m));
+            for (int q = 0; q < kTileThreads / kWave; ++q) m = dmax_ref(m, sh[q]);
+            // one address for all blocks: most find a larger value there already, and
+            // their loads, unlike atomics, do not queue
+            auto* res = reinterpret_cast<unsigned long long*>(&A.resid[A.iter]);
+            const unsigned long long mb = (unsigned long long)__double_as_longlong(m);
+            if (__hip_atomic_load(res, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < mb) atomicMax(res, mb);
         }
     }
 }

@@ -1,0 +1,33 @@
+"""Tiled Jacobi sweeps with several planes in flight: fewer planes than that, every
+remainder of a tile's planes, and densities under the floor of 1e-14, against the
+oracle's sweep.  Nine sweeps, each within about ten roundings (1.1e-15) of the
+oracle's, so 1e-14 and a factor of two."""
+import numpy as np
+import pytest
+
+from semiimplicitfv_amd import HLLCSolver, IdealGasEOS, JacobiPressureSolver, SemiImplicitSolver
+from tests.golden import problems
+from tests.helpers import rel_errs
+from tests.test_gpu_semi import _tile_problem
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("floor", [False, True])
+@pytest.mark.parametrize("shape", [(63, 4, 3), (64, 3, 4), (5, 9, 7), (65, 4, 21), (67, 6)])
+def test_jacobi_planes_in_flight(gpu, oracle_c, shape, floor):
+    periods = (0, 1, 1) if shape[-1] % 2 else (1, 0, 0)
+    cfg, mesh, rho, rhoc2, rhs, p0, dt = _tile_problem(shape, periods, seed=7 * sum(shape))
+    if floor:
+        mesh.interior(rho)[..., ::3] = 1e-16
+        rho = problems._fill_scalar_np(mesh, rho)
+    eos = IdealGasEOS(1.4, 1.0, cfg)
+    g = SemiImplicitSolver(mesh, HLLCSolver(eos), JacobiPressureSolver(), eos, None, cfg)
+    cpu = oracle_c.CpuSolver(mesh, cfg, 2, eos, "c")
+    pg, pc = p0.copy(), p0.copy()
+    hg, hc = np.zeros(9), np.zeros(9)
+    assert JacobiPressureSolver(g).solve(mesh, rho, rhoc2, rhs, pg, dt, 1e-300, 9, history=hg) == 9
+    assert cpu.jacobi(rho, rhoc2, rhs, pc, dt, 1e-300, 9, hc) == 9
+    l1, li = rel_errs(mesh.interior(pg), mesh.interior(pc))
+    assert l1 <= 2e-14 and li <= 2e-14, (l1, li)
+    g.close()
