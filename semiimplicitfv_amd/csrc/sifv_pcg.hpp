@@ -22,19 +22,17 @@
 // fields W[d]: W[d] at a cell holds the weight of its low face along d, and
 // the slot one past the last cell of a line holds the line's high boundary
 // face (0 on a wall, the wrap face of a periodic axis), so a row reads its
-// high weight from the next slot.  Each weight is the expression of the row
-// that owns the slot (the other row's operands in the same order), so
-// products equal those of recomputing the weights per row, up to the
-// compiler's choice of fused multiply-adds, without the 2*DIM FP64 divisions
-// per cell.  Scalars
+// high weight from the next slot.  The set-up, the coarse operators, the FP32
+// V-cycle and 1D read them; in 2D/3D the passes over the fine level form the
+// weights again from rho (RhoRow), which is less to read.  Scalars
 // (alpha, beta, the dot products) stay on the device; each product and update
 // kernel writes per-block partial sums that a one-block kernel folds in fixed
 // order, so a solve is deterministic run to run.  A device flag ends the
 // iteration: the host enqueues iterations in chunks and polls the flag.
 //
 // Per iteration, per interior cell: pcg_matvec (read p with its 2*DIM
-// neighbours, W, s; write q: 24 + 8 DIM B), pcg_update (read x p r q d s,
-// write x r z: 72 B), pcg_dir (read z p, write p: 24 B) -- 144 B/cell in 3D,
+// neighbours, rho, s; write q: 32 B in 2D/3D), pcg_update (read x p r q d s,
+// write x r z: 72 B), pcg_dir (read z p, write p: 24 B) -- 128 B/cell,
 // HBM-bound.
 #pragma once
 
@@ -176,15 +174,13 @@ __device__ __forceinline__ double pcg_row_f(const PcgArgs& A, V&& val, double si
 // XCDs) take a contiguous range of bricks, y fastest, so that neighbouring
 // bricks share that XCD's L2.  The block count is the elementwise kernels'
 // (their per-block partial sums keep one layout).
-#ifndef SIFV_PCG_BRICKS
-#define SIFV_PCG_BRICKS 1
-#endif
 constexpr int kBrickPlanes = 16;
 
-template <int DIM, typename F>
-__device__ __forceinline__ void pcg_bricks(const Grid& g, F&& body) {
+template <int DIM, int RY, typename F>
+__device__ __forceinline__ void pcg_columns(const Grid& g, F&& body) {
+    // body(i, j, k0, k1): column i of rows j .. j + RY - 1, also past the mesh's edges
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int bx = (g.nx + 63) / 64, by = (g.ny + 3) / 4;
+    const int bx = (g.nx + 63) / 64, by = (g.ny + 4 * RY - 1) / (4 * RY);
     const int bz = DIM == 3 ? (g.nz + kBrickPlanes - 1) / kBrickPlanes : 1;
     const long nbr = (long)bx * by * bz;
     const int G = (int)gridDim.x;
@@ -201,13 +197,124 @@ __device__ __forceinline__ void pcg_bricks(const Grid& g, F&& body) {
         const int cy = (int)(t % by);
         const long rest = t / by;
         const int cx = (int)(rest % bx), cz = (int)(rest / bx);
-        const int i = cx * 64 + tx, j = cy * 4 + ty;
-        if (i >= g.nx || j >= g.ny) continue;
         const int k0 = DIM == 3 ? cz * kBrickPlanes : 0;
         const int k1 = DIM == 3 ? min(g.nz, k0 + kBrickPlanes) : 1;
-        for (int k = k0; k < k1; ++k) body(i, j, k);
+        body(cx * 64 + tx, (cy * 4 + ty) * RY, k0, k1);
     }
 }
+
+// A row of S in a column (i, j) of a 2D/3D mesh with the face weights formed from the
+// densities: w = 4 area / ((rho + rho_nb)(h + h_nb)), the two faces of a direction
+// from one reciprocal.  The passes over the fine level are bound by memory, so 8 B of
+// rho instead of 24 B of weights (and instead of the diagonal's 8, where both are
+// needed) are worth the six faces' arithmetic.  What depends on the column alone is
+// kept over its planes, and density and v are carried from plane to plane.  A wall's
+// weight is 0 and its neighbour the cell itself.  At 256^3, from stored weights -> from
+// densities -> carried up the column: product 138 -> 140 -> 120 us, restriction
+// 174 -> 150 -> 135, post-smoothing 193 -> 186 -> 159.
+template <int DIM>
+struct RhoRow {
+    double gxl, gxr, gyl, gyr, hxy;
+    int pxl, pxr, pyl, pyr;   // offsets of the neighbours (wrapped)
+    int rxl, rxr, ryl, ryr;   // offsets of their densities (ghosts of wrapping faces are filled)
+    int il, ir, jl, jr;       // coordinates of the neighbours
+    double rm, rc, vm, vc;    // density and v of the plane below and of the next one, carried up the column
+    __device__ __forceinline__ RhoRow(const Grid& g, int i, int j) {
+        const double hx = g.dxw[i + g.ngx], hy = g.dyw[j + g.ngy];
+        hxy = 4.0 * hx * hy;
+        il = pcg_nbc(g, 0, 0, i);
+        ir = pcg_nbc(g, 0, 1, i);
+        jl = pcg_nbc(g, 1, 0, j);
+        jr = pcg_nbc(g, 1, 1, j);
+        const bool wxl = i == 0 && g.sbc[0] != BK_WRAP, wxr = i == g.nx - 1 && g.sbc[1] != BK_WRAP;
+        const bool wyl = j == 0 && g.sbc[2] != BK_WRAP, wyr = j == g.ny - 1 && g.sbc[3] != BK_WRAP;
+        gxl = wxl ? 0.0 : 4.0 * hy / (g.dxw[i - 1 + g.ngx] + hx);
+        gxr = wxr ? 0.0 : 4.0 * hy / (hx + g.dxw[i + 1 + g.ngx]);
+        gyl = wyl ? 0.0 : 4.0 * hx / (g.dyw[j - 1 + g.ngy] + hy);
+        gyr = wyr ? 0.0 : 4.0 * hx / (hy + g.dyw[j + 1 + g.ngy]);
+        pxl = il - i;
+        pxr = ir - i;
+        pyl = (jl - j) * g.nxT;
+        pyr = (jr - j) * g.nxT;
+        rxl = wxl ? 0 : -1;
+        rxr = wxr ? 0 : 1;
+        ryl = wyl ? 0 : -g.nxT;
+        ryr = wyr ? 0 : g.nxT;
+    }
+    // the column's first plane, v by val(index, i, j, k)
+    template <typename V>
+    __device__ __forceinline__ void begin(const PcgArgs& A, V&& val, int i, int j, int k) {
+        const Grid& g = A.g;
+        const size_t id = cell_index(g, i, j, k);
+        rm = rc = A.rho[id];
+        vm = vc = val(id, i, j, k);
+        if (DIM >= 3) {
+            const long sz = (long)g.nxT * g.nyT;
+            const int kl = pcg_nbc(g, 2, 0, k);
+            if (k > 0 || g.sbc[4] == BK_WRAP) rm = A.rho[id - sz];
+            vm = val(id + (kl - k) * sz, i, j, kl);
+        }
+    }
+    // (S v) at the next plane k; vi: v there; dd: the diagonal
+    template <typename V>
+    __device__ __forceinline__ double row(const PcgArgs& A, V&& val, double si, int i, int j, int k, size_t id, double& vi,
+                                          double& dd) {
+        const Grid& g = A.g;
+        const double* __restrict__ rho = A.rho;
+        double sxl = rc + rho[id + rxl], sxr = rc + rho[id + rxr];
+        double syl = rc + rho[id + ryl], syr = rc + rho[id + ryr];
+        double szl = 1.0, szr = 1.0, nzl = 0.0, nzr = 0.0, hl = 1.0, hr = 1.0;
+        vi = vc;
+        const double vxl = val(id + pxl, il, j, k), vxr = val(id + pxr, ir, j, k);
+        const double vyl = val(id + pyl, i, jl, k), vyr = val(id + pyr, i, jr, k);
+        double vzr = 0.0, rp = 0.0;
+        const double vzl = vm;
+        const double hz = g.dzw[k + g.ngz];
+        if (DIM >= 3) {
+            const long sz = (long)g.nxT * g.nyT;
+            const int kr = pcg_nbc(g, 2, 1, k);
+            const bool wl = k == 0 && g.sbc[4] != BK_WRAP, wr = k == g.nz - 1 && g.sbc[5] != BK_WRAP;
+            rp = rho[id + (wr ? 0 : sz)];
+            szl = rc + rm;
+            szr = rc + rp;
+            nzl = wl ? 0.0 : hxy;
+            nzr = wr ? 0.0 : hxy;
+            hl = g.dzw[k - 1 + g.ngz] + hz;
+            hr = hz + g.dzw[k + 1 + g.ngz];
+            vzr = val(id + (kr - k) * sz, i, j, kr);
+        }
+        // densities under the floor are rare: look once for all faces (a NaN is under
+        // nothing, and stays)
+        double lo = fmin(fmin(sxl, sxr), fmin(syl, syr));
+        if (DIM >= 3) lo = fmin(lo, fmin(szl, szr));
+        if (__builtin_expect(lo < 2e-14, 0)) {
+            sxl = dmax_ref(sxl, 2e-14);
+            sxr = dmax_ref(sxr, 2e-14);
+            syl = dmax_ref(syl, 2e-14);
+            syr = dmax_ref(syr, 2e-14);
+            szl = dmax_ref(szl, 2e-14);
+            szr = dmax_ref(szr, 2e-14);
+        }
+        double acc = si * vi;
+        dd = si;
+        auto faces = [&](double a, double b, double ga, double gb, double va, double vb) __attribute__((always_inline)) {
+            const double r = rcp_nr(a * b);
+            const double wa = ga * (b * r), wb = gb * (a * r);
+            acc += wa * (vi - va);
+            acc += wb * (vi - vb);
+            dd += wa;
+            dd += wb;
+        };
+        faces(sxl, sxr, gxl * hz, gxr * hz, vxl, vxr);
+        faces(syl, syr, gyl * hz, gyr * hz, vyl, vyr);
+        if (DIM >= 3) faces(szl * hl, szr * hr, nzl, nzr, vzl, vzr);
+        rm = rc;
+        rc = rp;
+        vm = vc;
+        vc = vzr;
+        return acc;
+    }
+};
 
 // Face weights W (low face of each cell; high face of the last cell of a
 // line in the slot after it), mass term s = V/c and diagonal d, from rho and
@@ -337,17 +444,29 @@ __global__ void __launch_bounds__(256) pcg_matvec_kernel(PcgArgs A) {
     __shared__ double sh[256 / kWave];
     const Grid& g = A.g;
     double pq = 0.0;
-    auto cell = [&](int i, int j, int k) {
-        const size_t id = cell_index(g, i, j, k);
-        const double qv = pcg_row<DIM>(A, A.p, A.s[id], i, j, k, id);
-        A.q[id] = qv;
-        pq += A.p[id] * qv;
-    };
-    if (DIM >= 2 && SIFV_PCG_BRICKS) {
-        pcg_bricks<DIM>(g, cell);
+    if constexpr (DIM >= 2) {
+        const double* __restrict__ p = A.p;
+        auto val = [&](size_t n, int, int, int) __attribute__((always_inline)) { return p[n]; };
+        pcg_columns<DIM, 1>(g, [&](int i, int j, int k0, int k1) {
+            if (i >= g.nx || j >= g.ny) return;
+            RhoRow<DIM> R(g, i, j);
+            R.begin(A, val, i, j, k0);
+            for (int k = k0; k < k1; ++k) {
+                const size_t id = cell_index(g, i, j, k);
+                double pv, dd;
+                const double qv = R.row(A, val, A.s[id], i, j, k, id, pv, dd);
+                A.q[id] = qv;
+                pq += pv * qv;
+            }
+        });
     } else {
         int i, j, k;
-        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k);
+        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) {
+            const size_t id = cell_index(g, i, j, k);
+            const double qv = pcg_row<DIM>(A, A.p, A.s[id], i, j, k, id);
+            A.q[id] = qv;
+            pq += A.p[id] * qv;
+        }
     }
     pcg_partials(A, sh, 1, pq, 0.0, 0.0);
 }
@@ -454,9 +573,9 @@ __global__ void __launch_bounds__(256) pcg_dir_kernel(PcgArgs A) {
 // for 1D, 2D, 3D.  Each step is linear and symmetric, so the preconditioner
 // is a fixed SPD operator and conjugate gradients stay valid.
 // Fine-level work per V-cycle and cell: pre (q = om r / d, folded into
-// pcg_update_kernel inside the iteration), restrict (read q with neighbours,
-// W, s, r: 48 B in 3D), prolong and post in one pass (read q W s r d and the
-// parent's correction, write z, with the r.z partial sums: 64 B).
+// pcg_update_kernel inside the iteration), restrict (read q and rho with
+// neighbours, s, r: 32 B in 2D/3D), prolong and post in one pass (read q rho s r
+// and the parent's correction, write z, with the r.z partial sums: 40 B).
 constexpr int kMgMaxLevels = 24;
 constexpr int kMgCoarseSweeps = 16;
 
@@ -469,10 +588,9 @@ __host__ __device__ constexpr double mg_omega(int dim) {
 // an FP32 pre-smoothed vector written by the CG update and FP32 coarse levels,
 // in FP32 arithmetic, while the conjugate-gradient recurrences, the product,
 // the dot products and the stopping test stay FP64.  The preconditioner is
-// then the V-cycle of the rounded operator evaluated in FP32: symmetric and
-// positive definite up to the FP32 rounding of each application.  Its
-// fine-level passes move 28 (restrict) and 40 (post) B per cell instead of 48
-// and 64.
+// then the V-cycle of the rounded operator evaluated in FP32 from stored FP32
+// weights: symmetric and positive definite up to the FP32 rounding of each
+// application.  Its fine-level passes move 28 (restrict) and 40 (post) B per cell.
 template <typename R>
 struct MgLevelT {
     int n[3];
@@ -625,6 +743,33 @@ __global__ void __launch_bounds__(256) mg_restrict_fine_kernel(MgArgsT<R> M) {
     const PcgArgs& A = M.A;
     const Grid& g = A.g;
     const MgLevelT<R>& C = M.C;
+    if constexpr (DIM >= 2 && sizeof(R) == 8) {
+        // a thread sums the children of its column in two rows and two planes, its
+        // neighbour lane adds the other column's
+        const double* __restrict__ q = A.q;
+        auto val = [&](size_t n, int, int, int) __attribute__((always_inline)) { return q[n]; };
+        pcg_columns<DIM, 2>(g, [&](int i, int j, int k0, int k1) {
+            const bool on = i < g.nx && j < g.ny;
+            const int ic = min(i, g.nx - 1), ja = min(j, g.ny - 1), jb = min(j + 1, g.ny - 1);
+            RhoRow<DIM> Ra(g, ic, ja), Rb(g, ic, jb);
+            Ra.begin(A, val, ic, ja, k0);
+            Rb.begin(A, val, ic, jb, k0);
+            for (int k = k0; k < k1; k += 2) {
+                double acc = 0.0;
+                for (int kk = k; kk < k + 2 && kk < k1; ++kk) {
+                    double qi, dd;
+                    const size_t ida = cell_index(g, ic, ja, kk), idb = cell_index(g, ic, jb, kk);
+                    acc += A.r[ida] - Ra.row(A, val, A.s[ida], ic, ja, kk, ida, qi, dd);
+                    const double rb = A.r[idb] - Rb.row(A, val, A.s[idb], ic, jb, kk, idb, qi, dd);
+                    if (j + 1 < g.ny) acc += rb;
+                }
+                const double other = __shfl_xor(acc, 1);
+                if (i + 1 < g.nx) acc += other;
+                if (on && (i & 1) == 0) C.b[mg_idx(C, i >> 1, j >> 1, k >> 1)] = acc;
+            }
+        });
+        return;
+    }
     const float* __restrict__ q32 = M.f32.q;
     auto q32v = [&](size_t id, int, int, int) __attribute__((always_inline)) { return q32[id]; };
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < C.cells; c += gridDim.x * blockDim.x) {
@@ -661,7 +806,11 @@ __global__ void __launch_bounds__(256) mg_post_fine_kernel(MgArgsT<R> M) {
     constexpr double om = mg_omega(DIM);
     const R* __restrict__ tc = C.t;
     double rz = 0.0;
-    auto cell = [&](int i, int j, int k) {
+    const double* __restrict__ q64 = A.q;
+    auto qp64 = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
+        return q64[n] + (double)tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
+    };
+    auto cell = [&](int i, int j, int k, RhoRow<DIM>* R2) __attribute__((always_inline)) {
         const size_t id = cell_index(g, i, j, k);
         const double r = A.r[id];
         double z;
@@ -674,23 +823,30 @@ __global__ void __launch_bounds__(256) mg_post_fine_kernel(MgArgsT<R> M) {
             const float a = face_row<DIM, float>(g, M.f32.W, qp, M.f32.s[id], i, j, k, id, qi);
             z = (double)(qi + (float)om * ((float)r - a) / M.f32.d[id]);
         } else {
-            const double* __restrict__ q = A.q;
-            auto qp = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
-                return q[n] + tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
-            };
-            double qi;
-            const double a = pcg_row_f<DIM>(A, qp, A.s[id], i, j, k, id, qi);
-            z = qi + om * (r - a) / A.d[id];
+            double qi, dd;
+            double a;
+            if constexpr (DIM >= 2) {
+                a = R2->row(A, qp64, A.s[id], i, j, k, id, qi, dd);
+            } else {
+                a = pcg_row_f<DIM>(A, qp64, A.s[id], i, j, k, id, qi);
+                dd = A.d[id];
+            }
+            z = qi + om * (r - a) / dd;
         }
         A.z[id] = z;
         rz += r * z;
         if (M.init) A.p[id] = z;
     };
-    if (DIM >= 2 && SIFV_PCG_BRICKS) {
-        pcg_bricks<DIM>(g, cell);
+    if constexpr (DIM >= 2) {
+        pcg_columns<DIM, 1>(g, [&](int i, int j, int k0, int k1) {
+            if (i >= g.nx || j >= g.ny) return;
+            RhoRow<DIM> R2(g, i, j);
+            if constexpr (sizeof(R) == 8) R2.begin(A, qp64, i, j, k0);
+            for (int k = k0; k < k1; ++k) cell(i, j, k, &R2);
+        });
     } else {
         int i, j, k;
-        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k);
+        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k, nullptr);
     }
     const double t = wave_sum(rz);
     const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
