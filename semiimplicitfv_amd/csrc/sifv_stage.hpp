@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "sifv_device.hpp"
+#include "sifv_shapes.hpp"
 
 #ifndef SIFV_PREFETCH_ROW_D
 #define SIFV_PREFETCH_ROW_D true
@@ -932,6 +933,7 @@ stage_xy_kernel(StageParams<T> P) {
     // registers at the top of the row, measured 5 % slower with the ring).
     constexpr bool RING = YDIR && PF && !PU && MODE == MODE_FULL && NPH == 0;
     constexpr int RN = R + 1;
+    static_assert(ring_slot(first_ring_row(R), RN) >= 0, "first row of the ring");
     constexpr int NCVR = DIM + 2 + 2 * NPH;
     __shared__ T sUr[RING ? RN : 1][RING ? NCVR : 1][kWave];
 
@@ -950,7 +952,7 @@ stage_xy_kernel(StageParams<T> P) {
             if constexpr (PF) {
                 raw_to_cell<DIM, NPH, T>(P, nextRow, win[R - 1]);
                 if constexpr (RING) {
-                    const int slot = (r + R) % RN;
+                    const int slot = ring_slot(r + R, RN);
 #pragma unroll
                     for (int q = 0; q < NCVR; ++q) sUr[slot][q][lane] = nextRow.U[q];
                 }
@@ -1111,7 +1113,7 @@ stage_xy_kernel(StageParams<T> P) {
                     T uring[NCVR];
                     if (r > Y0) {
 #pragma unroll
-                        for (int q = 0; q < NCVR; ++q) uring[q] = sUr[r % RN][q][lane];
+                        for (int q = 0; q < NCVR; ++q) uring[q] = sUr[ring_slot(r, RN)][q][lane];
                     } else {
 #pragma unroll
                         for (int q = 0; q < NCVR; ++q) uring[q] = *field_at(P.src, P.total, q, id);
@@ -1198,6 +1200,7 @@ stage_z_kernel(StageParams<T> P) {
     // the update reads them (instead of a second read from HBM)
     constexpr int NCV = DIM + 2 + 2 * NPH;
     constexpr int RING = R + 1;
+    static_assert(ring_slot(first_ring_row(R) - 1, RING) >= 0, "first plane of the ring");
     __shared__ T sU[RING][NCV][kWave];
 #pragma unroll
     for (int w = 1; w < WS; ++w) {
@@ -1206,7 +1209,7 @@ stage_z_kernel(StageParams<T> P) {
             RawCell<DIM, NPH, T> rc;
             load_row<DIM, NPH, T>(P, P.src, cm, j, kk, rc);
 #pragma unroll
-            for (int q = 0; q < NCV; ++q) sU[(kk + RING) % RING][q][lane] = rc.U[q];
+            for (int q = 0; q < NCV; ++q) sU[ring_slot(kk, RING)][q][lane] = rc.U[q];
             raw_to_cell<DIM, NPH, T>(P, rc, win[w]);
         } else {
             RawCell<DIM, NPH, T> rc;
@@ -1225,14 +1228,14 @@ stage_z_kernel(StageParams<T> P) {
         }
         if constexpr (PF) {
 #pragma unroll
-            for (int q = 0; q < NCV; ++q) sU[(r + R + RING) % RING][q][lane] = nextRow.U[q];
+            for (int q = 0; q < NCV; ++q) sU[ring_slot(r + R, RING)][q][lane] = nextRow.U[q];
             raw_to_cell<DIM, NPH, T>(P, nextRow, win[WS - 1]);
             if (r + 1 < Z1) load_row<DIM, NPH, T>(P, P.src, cm, j, r + 1 + R, nextRow);
         } else {
             RawCell<DIM, NPH, T> rc;
             load_row<DIM, NPH, T>(P, P.src, cm, j, r + R, rc);
 #pragma unroll
-            for (int q = 0; q < NCV; ++q) sU[(r + R + RING) % RING][q][lane] = rc.U[q];
+            for (int q = 0; q < NCV; ++q) sU[ring_slot(r + R, RING)][q][lane] = rc.U[q];
             raw_to_cell<DIM, NPH, T>(P, rc, win[WS - 1]);
         }
         sigwin[WS - 1] = useSig ? (T)load_sigma<DIM>(P, cc, j, r + R) : T(0);
@@ -1266,7 +1269,7 @@ stage_z_kernel(StageParams<T> P) {
             const double h[3] = {dxc, dyj, dzr};
             T Upre[NCV];
 #pragma unroll
-            for (int q = 0; q < NCV; ++q) Upre[q] = sU[(r + RING) % RING][q][lane];
+            for (int q = 0; q < NCV; ++q) Upre[q] = sU[ring_slot(r, RING)][q][lane];
             double dc = finish_cell<DIM, NPH, SEMI, T, true, C>(P, id, acc, win[WROW], h, dt, P.dtPartial != nullptr,
                                                                 Upre);
             dtMin = dmin_ref(dtMin, dc);
