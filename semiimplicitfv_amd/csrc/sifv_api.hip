@@ -322,53 +322,22 @@ int ensure_partials(sifv_handle* h, int n) {
 // ---- stage launch ---------------------------------------------------------
 int recon_radius(int order) { return required_ghosts(order); }
 
-void stage_shape(const sifv_handle* h, int& nstrip, int& nseg, int& rows) {
-    nstrip = (h->nx + kOwn - 1) / kOwn;
-    if (h->dim == 1) {
-        nseg = 1;
-        rows = 1;
-        return;
-    }
-    long planes = h->dim == 3 ? h->nz : 1;
-    if (h->rowsOverride > 0) {
-        rows = h->rowsOverride;
-    } else {
-        // aim for >= ~8k waves so every CU holds several waves (2D: ~16k,
-        // 16 rows per wave at 4096^2, the fastest of 8..128 rows measured for
-        // both the FP64 and the FP32-bulk kernels); meshes too small for 8 rows
-        // per wave at that count get about one wave per SIMD slot (3072 at three
-        // waves per SIMD) with 4..8 rows, trading the 2-row warm-up against
-        // filling the chip (1024^2: 6 rows, measured fastest of 4..16)
-        long target = h->dim == 2 ? 16384 : 8192;
-        const long cols = (long)h->ny * nstrip * planes;
-        long r = cols / target;
-        if (r >= 8) {
-            rows = 8;
-            while (rows < 64 && rows * 2 <= r) rows *= 2;
-        } else {
-            rows = (int)std::max<long>(4, std::min<long>(8, (cols + 3071) / 3072));
-        }
-    }
-    rows = std::min(rows, h->ny);
-    nseg = (h->ny + rows - 1) / rows;
+// Strips, segments and rows per wave of a stage's march (the x+y pass in 3D).
+StageShape march_shape(const sifv_handle* h) {
+    return march_shape_of(h->dim, h->nx, h->ny, h->nz, h->rowsOverride);
 }
 
-// Waves per workgroup of the 2D tile kernel (sifv_tile.hpp) for an explicit
-// stage, or 0 for the marching kernel.  Meshes whose marching waves cannot fill
-// the chip take tiles: a wave's serial chain of 6 rows costs 22 us there, a
-// tile 11 us (128^2 FP64; 128^2 water/air 44 -> 16 us, FP32 21 -> 10 us).  The
-// line is where the tiles' halo rows and barriers cost more than that:
-// 576^2 30.4 against 34.9 us and 640^2 36.8 against 35.4 (FP64), 768^2 28.6
-// against 31.7 and 896^2 37.6 against 36.7 (FP32), 800^2 99 against 102
-// (water/air).  Small tiles (2 rows) while those of 8 rows would leave half
-// the 256 CUs idle: 128^2 10.8 against 12.8 us, 320^2 16.0 against 13.7.
-int stage_tile_waves(const sifv_handle* h, bool fp32) {
-    if (h->dim != 2 || h->rowsOverride > 0 || recon_radius(h->cfg.reconOrder) != 3) return 0;
-    if (fp32 && h->nph) return 0;
-    const long cells = (long)h->nx * h->ny;
-    if (cells > (h->nph ? 640000 : fp32 ? 600000 : 360000)) return 0;
-    const long blocks = (long)((h->nx + kOwn - 1) / kOwn) * ((h->ny + kTileWaves - 3) / (kTileWaves - 2));
-    return blocks < 128 ? kTileSmall : kTileWaves;
+// The same of an explicit stage, whose full 2D form may run on tiles.
+StageShape explicit_stage_shape(const sifv_handle* h) {
+    const bool tiles = h->dim == 2 && h->rowsOverride <= 0 && recon_radius(h->cfg.reconOrder) == 3;
+    const int tw = tiles ? tile_waves_of(h->nx, h->ny, h->nph, h->precision != SIFV_FP64) : 0;
+    return tw ? tile_shape_of(h->nx, h->ny, tw) : march_shape(h);
+}
+
+// Blocks (dt partials) of the stress limits' reduction.
+int stress_blocks(const sifv_handle* h) {
+    const size_t ncell = (size_t)h->nx * h->ny * h->nz;
+    return (int)std::min<size_t>((ncell + kRedThreads - 1) / kRedThreads, kStressPartials);
 }
 
 void zpass_shape(const sifv_handle* h, int& nstrip, int& nseg, int& rows) {
@@ -554,26 +523,19 @@ int launch_stage_p(sifv_handle* h, const T* srcp, const T* u0p, T* dstp, const d
     StageKernels<T> k = stage_kernels<T>(h, semi);
     if (!k.xy || (h->dim == 3 && !k.z)) return fail(SIFV_ERR_UNSUPPORTED, "no stage kernel for this configuration");
     const bool wantDt = last && !semi && h->cfg.explicitParams.constDt <= 0.0;
-    int nstrip, nseg, rows;
-    stage_shape(h, nstrip, nseg, rows);
-    P.rows = rows;
-    P.nseg = nseg;
-    P.nstrip = nstrip;
-    int nb = nstrip * nseg * (h->dim == 3 ? h->nz : 1);
-    const int tw = semi ? 0 : stage_tile_waves(h, sizeof(T) == 4);
-    if (tw) {
-        k.xy = stage_tile_for<T>(h->riemann, h->nph, stage_lean(h->cfg), tw);
-        P.rows = tw - 2;
-        P.nseg = (h->ny + P.rows - 1) / P.rows;
-        nb = nstrip * P.nseg;
-    }
+    const StageShape shape = semi ? march_shape(h) : explicit_stage_shape(h);
+    P.rows = shape.rows;
+    P.nseg = shape.nseg;
+    P.nstrip = shape.nstrip;
+    const int nb = shape.blocks(h->dim == 3 ? h->nz : 1);
+    const int tw = shape.tileWaves;
+    if (tw) k.xy = stage_tile_for<T>(h->riemann, h->nph, stage_lean(h->cfg), tw);
     // viscous / capillary limits of the new state: their own reduction after
     // the stage, into the partial slots after the fused acoustic minima
     const double viscMu = h->cfg.viscousMu > 0.0 ? h->cfg.viscousMu : 0.0;
     const double capSigma = has_surface_tension(h->cfg) ? h->cfg.surfaceTensionSigma : 0.0;
     const bool stressDt = wantDt && (viscMu > 0.0 || capSigma > 0.0);
-    const size_t ncell = (size_t)h->nx * h->ny * h->nz;
-    const int nbs = stressDt ? (int)std::min<size_t>((ncell + kRedThreads - 1) / kRedThreads, 2048) : 0;
+    const int nbs = stressDt ? stress_blocks(h) : 0;
     P.dtPartial = nullptr;
     if (wantDt && h->dim < 3) {
         int rc = ensure_partials(h, nb + nbs);
@@ -2353,7 +2315,6 @@ int advance_impl(sifv_handle* h, const sifv_config* cfg, int nsteps, double endT
 // GPU (overlapping calls on one GPU race on it).  Nothing has to start at
 // zero: every partial the dt finalize reads was written earlier in the same
 // step.  Host code uses only the per-device address from hipGetSymbolAddress.
-constexpr int kScratchPartials = 65536;  // 512 KiB of FP64 block minima
 static __device__ __align__(256) double scratch[kScratchPartials];
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -2382,18 +2343,14 @@ int scratch_for(const sifv_handle* h, double** out) {
 // Largest number of dt partials one step of this handle writes.
 int partials_needed(const sifv_handle* h) {
     int need = elementwise_blocks(h);  // dt from the primitive arrays
-    int nstrip, nseg, rows;
-    stage_shape(h, nstrip, nseg, rows);
-    int stage = nstrip * nseg;
+    int stage = explicit_stage_shape(h).blocks(1);
     if (h->dim == 3) {
         int zs, zn, zr;
         zpass_shape(h, zs, zn, zr);
         stage = zs * zn * h->ny;
     }
     const bool stress = h->cfg.viscousMu > 0.0 || has_surface_tension(h->cfg);
-    const size_t ncell = (size_t)h->nx * h->ny * h->nz;
-    const int nbs = stress ? (int)std::min<size_t>((ncell + kRedThreads - 1) / kRedThreads, 2048) : 0;
-    return std::max(need, stage + nbs);
+    return std::max(need, stage + (stress ? stress_blocks(h) : 0));
 }
 }  // namespace
 

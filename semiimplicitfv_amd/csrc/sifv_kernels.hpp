@@ -32,7 +32,6 @@ StageKernels<float> stage_kernels_fp32_mp(int dim, int R, int rs);
 
 // Tile form of a full explicit 2D stage (R = 3): nw waves per workgroup
 // (kTileSmall or kTileWaves); null when there is none.
-constexpr int kTileSmall = 4, kTileWaves = 10;
 template <typename T>
 StageFn<T> stage_tile_for(int rs, int nph, bool lean, int nw);
 template <>

@@ -2,6 +2,8 @@
 // Standard C++ only, so that tests compile it with the host compiler.
 #pragma once
 
+#include <algorithm>
+
 namespace sifv {
 
 // Slot of a row (or plane) in a ring of n; the warm-up rows of a march start at
@@ -11,5 +13,70 @@ constexpr int ring_slot(int row, int n) { return (row + n) % n; }
 // First row (plane) a march puts into its ring of R + 1: row + R of the first
 // warm-up row of the first segment.
 constexpr int first_ring_row(int R) { return -2 + R; }
+
+constexpr int kOwn = 62;  // owned columns per wave in the x-marching and tile kernels
+constexpr int kTileSmall = 4, kTileWaves = 10;  // waves per workgroup of the 2D tile kernel
+
+// dt block minima: room of the allocation-free time loop (512 KiB of FP64), and
+// the most that the stress limits' reduction adds to a stage's own.
+constexpr int kScratchPartials = 65536;
+constexpr int kStressPartials = 2048;
+
+// Decomposition of a stage: strips of kOwn columns x segments of `rows` rows, a
+// wave each (a workgroup of tileWaves waves where that is not 0).
+struct StageShape {
+    int nstrip, nseg, rows, tileWaves;
+    int blocks(int planes) const { return nstrip * nseg * planes; }
+};
+
+inline StageShape march_shape_of(int dim, int nx, int ny, int nz, int rowsOverride) {
+    const int nstrip = (nx + kOwn - 1) / kOwn;
+    if (dim == 1) return StageShape{nstrip, 1, 1, 0};
+    const long planes = dim == 3 ? nz : 1;
+    int rows = rowsOverride;
+    if (rowsOverride <= 0) {
+        // aim for >= ~8k waves so every CU holds several waves (2D: ~16k,
+        // 16 rows per wave at 4096^2, the fastest of 8..128 rows measured for
+        // both the FP64 and the FP32-bulk kernels); meshes too small for 8 rows
+        // per wave at that count get about one wave per SIMD slot (3072 at three
+        // waves per SIMD) with 4..8 rows, trading the 2-row warm-up against
+        // filling the chip (1024^2: 6 rows, measured fastest of 4..16)
+        const long target = dim == 2 ? 16384 : 8192;
+        const long cols = (long)ny * nstrip * planes;
+        const long r = cols / target;
+        if (r >= 8) {
+            rows = 8;
+            while (rows < 64 && rows * 2 <= r) rows *= 2;
+        } else {
+            rows = (int)std::max<long>(4, std::min<long>(8, (cols + 3071) / 3072));
+        }
+    }
+    rows = std::min(rows, ny);
+    return StageShape{nstrip, (ny + rows - 1) / rows, rows, 0};
+}
+
+inline StageShape tile_shape_of(int nx, int ny, int waves) {
+    const int rows = waves - 2;
+    return StageShape{(nx + kOwn - 1) / kOwn, (ny + rows - 1) / rows, rows, waves};
+}
+
+// Waves per workgroup of the 2D tile kernel (sifv_tile.hpp) for an explicit
+// stage, or 0 for the marching kernel.  Meshes whose marching waves cannot fill
+// the chip take tiles: a wave's serial chain of 6 rows costs 22 us there, a
+// tile 11 us (128^2 FP64; 128^2 water/air 44 -> 16 us, FP32 21 -> 10 us).  The
+// line is where the tiles' halo rows and barriers cost more than that:
+// 576^2 30.4 against 34.9 us and 640^2 36.8 against 35.4 (FP64), 768^2 28.6
+// against 31.7 and 896^2 37.6 against 36.7 (FP32), 800^2 99 against 102
+// (water/air).  Small tiles (2 rows) while those of 8 rows would leave half
+// the 256 CUs idle: 128^2 10.8 against 12.8 us, 320^2 16.0 against 13.7.
+// A mesh of few columns whose tiles are more than the allocation-free loop has
+// dt partials for marches (1 x 600000 water/air: 75000 tiles).
+inline int tile_waves_of(int nx, int ny, int nph, bool fp32) {
+    if (fp32 && nph) return 0;
+    if ((long)nx * ny > (nph ? 640000 : fp32 ? 600000 : 360000)) return 0;
+    const int blocks = tile_shape_of(nx, ny, kTileWaves).blocks(1);
+    if (blocks > kScratchPartials - kStressPartials) return 0;
+    return blocks < 128 ? kTileSmall : kTileWaves;
+}
 
 }  // namespace sifv

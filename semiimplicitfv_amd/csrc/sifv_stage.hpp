@@ -57,7 +57,6 @@
 
 namespace sifv {
 
-constexpr int kOwn = 62;  // owned columns per wave in the x-marching kernels
 
 enum { MODE_FULL = 0, MODE_XY = 1 };
 

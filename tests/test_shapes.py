@@ -1,5 +1,5 @@
 """Index and shape arithmetic of csrc/sifv_shapes.hpp, compiled here with the host
-compiler: the LDS rings of the marching kernels."""
+compiler: the LDS rings of the marching kernels, the rule that picks stage tiles."""
 import ctypes as C
 import os
 import subprocess
@@ -12,6 +12,10 @@ SHIM = """
 extern "C" {
 int ring_slot(int row, int n) { return sifv::ring_slot(row, n); }
 int first_ring_row(int R) { return sifv::first_ring_row(R); }
+int tile_waves(int nx, int ny, int nph, int fp32) { return sifv::tile_waves_of(nx, ny, nph, fp32 != 0); }
+int tile_blocks(int nx, int ny, int tw) { return sifv::tile_shape_of(nx, ny, tw).blocks(1); }
+int scratch_partials() { return sifv::kScratchPartials; }
+int stress_partials() { return sifv::kStressPartials; }
 }
 """
 
@@ -35,3 +39,24 @@ def test_ring_slots_in_range_and_distinct(shapes, R):
     slots = [shapes.ring_slot(r, n) for r in range(R - 3, 40)]
     assert all(0 <= s < n for s in slots)
     assert all(len(set(slots[i:i + n])) == n for i in range(len(slots) - n + 1))
+
+
+@pytest.mark.parametrize("nph,fp32", [(0, 0), (2, 0), (0, 1), (2, 1)])
+def test_tiles_fit_the_allocation_free_partials(shapes, nph, fp32):
+    """A mesh on tiles leaves dt partials enough for the allocation-free loop, as its
+    march does (16384 waves and 2048 blocks of stress limits against 65536)."""
+    cap, stress = shapes.scratch_partials(), shapes.stress_partials()
+    tiled = 0
+    for nx in list(range(1, 70)) + [500, 4000, 80000, 640000]:
+        for ny in (1, 2, 9, 800, 5000, 300000, 360000, 507904, 524289, 600000, 640000):
+            tw = shapes.tile_waves(nx, ny, nph, fp32)
+            assert tw in (0, 4, 10)
+            if tw:
+                tiled += 1
+                assert shapes.tile_blocks(nx, ny, tw) + stress <= cap, (nx, ny)
+    assert (tiled == 0) == bool(nph and fp32)
+    # as many 8-row tiles as there is room for beside the stress limits, and one more
+    if nph or fp32:
+        ny = 8 * (cap - stress)
+        assert shapes.tile_waves(1, ny, nph, fp32) == (0 if nph and fp32 else 10)
+        assert shapes.tile_waves(1, ny + 1, nph, fp32) == 0

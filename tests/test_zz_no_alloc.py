@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 from semiimplicitfv_amd import ExplicitSolver, HLLCSolver, _abi, cases, uniform_mesh
-from tests.helpers import make_case
+from tests.helpers import make_case, make_two_phase_case
 
 pytestmark = pytest.mark.gpu
 
@@ -115,5 +115,25 @@ def test_noalloc_refusals(gpu):
     rc, _, _ = _noalloc(b, cfg, 1)
     assert rc == _abi.ERR_UNSUPPORTED
     b.timing(False)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("precision,two", [("fp64", True), ("mixed", False)])
+def test_noalloc_one_column(gpu, precision, two):
+    """600000 rows of one column: on 8-row tiles they would need 75000 dt partials,
+    more than the static array holds; the march they take needs 18750."""
+    def build():
+        if two:
+            cfg, mesh, st, eos = make_two_phase_case(2, (1, 600000), seed=9, p_jump=False)
+        else:
+            cfg, mesh, st, eos = make_case(2, (1, 600000), seed=9, shock=False)
+        return cfg, mesh, st, eos, HLLCSolver(eos)
+    cfg, mesh, a, b = _pair(build, precision)
+    ta, na = a.advance(cfg, 2, 1e30, 0.0)
+    rc, tb, nb = _noalloc(b, cfg, 2)
+    assert rc == 0, _abi.load_library().sifv_last_error()
+    assert (ta, na) == (tb, nb) and na == 2
+    _same(a, b, FIELDS2)
     a.close()
     b.close()
