@@ -136,6 +136,9 @@ __device__ __forceinline__ double rcp_nr(double x) {
     return fma(r, e, r);
 }
 
+// 1/x for any x >= 1e-290: 0 for an infinite x, where rcp_nr gives a NaN.
+__device__ __forceinline__ double rcp_inf(double x) { return x == __builtin_inf() ? 0.0 : rcp_nr(x); }
+
 // a / b and 1 / b, sqrt(x) for normal operands (see SIFV_FAST_DIV); the
 // quotient gets one residual correction q + r (a - b q).
 __device__ __forceinline__ double div_fast(double a, double b) {

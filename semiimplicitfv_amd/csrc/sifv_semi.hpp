@@ -681,6 +681,26 @@ __global__ void __launch_bounds__(kTileThreads) jacobi_tile_kernel(JacobiTileArg
                 off += cL * pzm + cR * pzp;
                 diag += cL + cR;
             }
+            if constexpr (F64) {
+                // an infinite density, or a product of two faces out of range, leaves
+                // a NaN: one reciprocal per face, 0 for an infinite density
+                if (__builtin_expect(!(diag >= 0.0), 0)) {
+                    off = diag = 0.0;
+                    auto face = [&](double sum, double d, double pn) __attribute__((always_inline)) {
+                        const double c = rcp_inf(sum * d);
+                        off += c * pn;
+                        diag += c;
+                    };
+                    face(sxl, dLx, xl.p);
+                    face(sxr, dRx, xr.p);
+                    face(syl, dLy, yl.p);
+                    face(syr, dRy, yr.p);
+                    if (z) {
+                        face(szl, dlz, pzm);
+                        face(szr, drz, pzp);
+                    }
+                }
+            }
             const size_t id = plane(k) + org;
             if constexpr (F64) {
                 const double co = q2 * dt2;

@@ -31,3 +31,24 @@ def test_jacobi_planes_in_flight(gpu, oracle_c, shape, floor):
     l1, li = rel_errs(mesh.interior(pg), mesh.interior(pc))
     assert l1 <= 2e-14 and li <= 2e-14, (l1, li)
     g.close()
+
+
+@pytest.mark.parametrize("shape", [(65, 9, 21), (64, 5, 4), (67, 6)])
+def test_jacobi_infinite_density(gpu, oracle_c, shape):
+    """Faces of a cell of infinite density have coefficient 0 and everything stays
+    finite: single cells, neighbouring ones, and one at a wall and a wrapping face."""
+    cfg, mesh, rho, rhoc2, rhs, p0, dt = _tile_problem(shape, (1, 0, 0), seed=5 * sum(shape))
+    mesh.interior(rho)[..., ::3, 5::7] = np.inf
+    mesh.interior(rho)[..., 1, 11:13] = np.inf
+    mesh.interior(rho)[..., 0, 0] = np.inf
+    rho = problems._fill_scalar_np(mesh, rho)
+    eos = IdealGasEOS(1.4, 1.0, cfg)
+    g = SemiImplicitSolver(mesh, HLLCSolver(eos), JacobiPressureSolver(), eos, None, cfg)
+    cpu = oracle_c.CpuSolver(mesh, cfg, 2, eos, "c")
+    pg, pc = p0.copy(), p0.copy()
+    assert JacobiPressureSolver(g).solve(mesh, rho, rhoc2, rhs, pg, dt, 1e-300, 9) == 9
+    assert cpu.jacobi(rho, rhoc2, rhs, pc, dt, 1e-300, 9, np.zeros(9)) == 9
+    assert np.isfinite(mesh.interior(pc)).all()
+    l1, li = rel_errs(mesh.interior(pg), mesh.interior(pc))
+    assert l1 <= 2e-14 and li <= 2e-14, (l1, li)
+    g.close()
