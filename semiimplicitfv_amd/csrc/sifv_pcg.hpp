@@ -308,6 +308,25 @@ struct RhoRow {
         faces(sxl, sxr, gxl * hz, gxr * hz, vxl, vxr);
         faces(syl, syr, gyl * hz, gyr * hz, vyl, vyr);
         if (DIM >= 3) faces(szl * hl, szr * hr, nzl, nzr, vzl, vzr);
+        // an infinite density, or a product of two faces out of range, leaves a NaN:
+        // one reciprocal per face, 0 for an infinite density
+        if (__builtin_expect(!(dd >= 0.0), 0)) {
+            acc = si * vi;
+            dd = si;
+            auto face = [&](double a, double ga, double va) __attribute__((always_inline)) {
+                const double w = ga * rcp_inf(a);
+                acc += w * (vi - va);
+                dd += w;
+            };
+            face(sxl, gxl * hz, vxl);
+            face(sxr, gxr * hz, vxr);
+            face(syl, gyl * hz, vyl);
+            face(syr, gyr * hz, vyr);
+            if (DIM >= 3) {
+                face(szl * hl, nzl, vzl);
+                face(szr * hr, nzr, vzr);
+            }
+        }
         rm = rc;
         rc = rp;
         vm = vc;

@@ -45,3 +45,27 @@ def test_pcg_rows_from_densities(gpu, oracle_c, shape, periods, floor, kind):
     assert 0 < ig < 2000 and abs(ig - ic) <= max(2, ic // 10), (ig, ic)
     ref = mesh.interior(pc)
     assert np.abs(mesh.interior(pg) - ref).max() <= 1e3 * tol * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("kind", ["PCG", "MGPCG"])
+@pytest.mark.parametrize("shape,periods", [((65, 9, 17), (0, 1, 0)), ((66, 7, 1), (1, 0, 0))])
+def test_pcg_infinite_density(gpu, oracle_c, shape, periods, kind):
+    """Faces of a cell of infinite density have weight 0 and everything stays finite;
+    the bars of test_pcg_rows_from_densities."""
+    cfg, mesh, rho, rhoc2, rhs, dt = _system(shape, periods, False)
+    mesh.interior(rho)[..., ::3, 5::7] = np.inf
+    mesh.interior(rho)[..., 1, 11:13] = np.inf
+    mesh.interior(rho)[..., 0, 0] = np.inf
+    rho = problems._fill_scalar_np(mesh, rho)
+    tol = 1e-7
+    eos = IdealGasEOS(1.4, 1.0, cfg)
+    g = SemiImplicitSolver(mesh, HLLCSolver(eos), SOLVERS[kind](), eos, None, cfg)
+    pg, pc = np.zeros(mesh.totalCells()), np.zeros(mesh.totalCells())
+    ig = SOLVERS[kind](g).solve(mesh, rho, rhoc2, rhs, pg, dt, tol, 2000)
+    g.close()
+    cpu = oracle_c.CpuSolver(mesh, cfg, 2, eos, "c")
+    ic = (cpu.pcg if kind == "PCG" else cpu.mgpcg)(rho, rhoc2, rhs, pc, dt, tol, 2000)
+    assert 0 < ig < 2000 and abs(ig - ic) <= max(2, ic // 10), (ig, ic)
+    ref = mesh.interior(pc)
+    assert np.isfinite(ref).all()
+    assert np.abs(mesh.interior(pg) - ref).max() <= 1e3 * tol * np.abs(ref).max()
