@@ -217,6 +217,7 @@ struct sifv_handle {
     int igrStrips = 0, igrPeriod = 0, igrSlots = 0;
     double* igrRec = nullptr;
     unsigned long long* igrEdge = nullptr;
+    long long igrWaitTicks = 0; // longest wait of a strip, in ticks of the device's wall clock
     unsigned igrTag = 1;        // tag of the next solve's initial edge values
     int* igrFlags = nullptr;   // [ntiles] tile epochs, [ntiles] error flag
     int igrNtx = 0, igrNty = 0, igrTj = 1, igrTiles = 0;
@@ -1661,6 +1662,9 @@ int setup_igr(sifv_handle* h) {
             HIPCHK(hipMalloc(&h->igrEdge, ne));
             HIPCHK(hipMemset(h->igrEdge, 0, ne));
             h->igrTag = 1;
+            int khz = 0;
+            HIPCHK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, h->device));
+            h->igrWaitTicks = strip_wait_ticks(khz);
         }
     }
     return SIFV_OK;
@@ -1737,6 +1741,7 @@ int run_igr(sifv_handle* h, int src, const int* active) {
         SA.nsweeps = iters;
         SA.perX = h->sbc[0] == BK_WRAP;
         SA.perY = h->sbc[2] == BK_WRAP;
+        SA.waitTicks = h->igrWaitTicks;
         void* sargs2[] = {&SA};
         rc = timed_launch(h, reinterpret_cast<const void*>(K.sweep), dim3(h->igrStrips), dim3(kStripWaves * kWave), sargs2);
         if (rc) return rc;

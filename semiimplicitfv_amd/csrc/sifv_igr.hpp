@@ -501,6 +501,7 @@ struct IgrStripArgs {
     int W, P, nsweeps;
     int ns;                // record slots per strip; P is a multiple of it
     int perX, perY;
+    long long waitTicks;   // longest wait, in ticks of the device's wall clock
 };
 
 __device__ __forceinline__ double dpp_shl1(double v) {   // lane l <- lane l+1
@@ -536,7 +537,9 @@ __device__ __forceinline__ double dpp_shl1_in(double v, double edge) {
 // the step that stored its sigma; wave 0 has at most seven groups of stores
 // outstanding when it counts a group as done, so that store is complete for every
 // P >= 129 (waiting for all but two groups made the stores' latency the limit).
-// Every wait is bounded and ends on the abort flag.
+// Every wait is bounded, by time (strips may wait for CUs that another stream's
+// kernels hold, and a pass of a wave that polls LDS is some 50 ns), and ends on the
+// abort flag.
 constexpr int kStripRecGroups = 5;
 constexpr int kStripWaves = 7;
 constexpr int kStripRing = 192;   // steps of wave 0's results and inputs held in LDS
@@ -570,15 +573,22 @@ __global__ void __launch_bounds__(64 * kStripWaves) igr_strip_kernel(IgrStripArg
     // the helper waves watch the device error flag and raise the block's abort
     // flag, which waves 0 and 3 poll in LDS
     auto aborted = [&]() __attribute__((always_inline)) { return __hip_atomic_load(&sFlag[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0; };
-    // one idle pass of a helper wave; true: give up
+    // true when a wait whose first look was at `since` has been too long
+    auto late = [&](int looks, long long& since) __attribute__((always_inline)) {
+        const long long t = wall_clock64();
+        if (looks == 1) since = t;
+        return t - since > A.waitTicks;
+    };
+    // one idle pass of a helper wave (idle: passes since it last moved); true: give up
+    long long since = 0;
     auto idle_pass = [&](int& idle) __attribute__((always_inline)) {
-        const bool budget = ++idle > (1 << 25);
-        if (budget) __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (aborted() || ((idle & 255) == 0 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
-            __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            return true;
+        bool stop = aborted();
+        if ((++idle & 255) == 0) {
+            if (late(idle >> 8, since)) __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            stop = stop || __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
         }
-        return budget;
+        if (stop) __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return stop;
     };
     if (wave == 4) {
         int pub = 0, idle = 0;
@@ -801,7 +811,7 @@ __global__ void __launch_bounds__(64 * kStripWaves) igr_strip_kernel(IgrStripArg
             const int l = peek(0), d = peek(7), p = peek(2), ab = peek(3);
             count(l, d, p);
             if (__builtin_amdgcn_readfirstlane(ab) != 0) return false;
-            if (++spins > (1 << 27)) {
+            if ((++spins & 0xffff) == 0 && late(spins >> 16, since)) {
                 __hip_atomic_store(A.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&sFlag[3], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 return false;

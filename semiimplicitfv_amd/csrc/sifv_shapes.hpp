@@ -79,4 +79,8 @@ inline int tile_waves_of(int nx, int ny, int nph, bool fp32) {
     return blocks < 128 ? kTileSmall : kTileWaves;
 }
 
+// Longest wait of a strip of the IGR sweep for another one, 30 s, in ticks of a clock
+// of `khz` (the device's wall clock: 100 MHz, also where the rate is not told).
+constexpr long long strip_wait_ticks(int khz) { return 30LL * 1000 * (khz > 0 ? khz : 100000); }
+
 }  // namespace sifv

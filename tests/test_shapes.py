@@ -1,5 +1,6 @@
 """Index and shape arithmetic of csrc/sifv_shapes.hpp, compiled here with the host
-compiler: the LDS rings of the marching kernels, the rule that picks stage tiles."""
+compiler: the LDS rings of the marching kernels, the rule that picks
+stage tiles, the bound of the IGR strips' waits."""
 import ctypes as C
 import os
 import subprocess
@@ -15,6 +16,7 @@ int first_ring_row(int R) { return sifv::first_ring_row(R); }
 int tile_waves(int nx, int ny, int nph, int fp32) { return sifv::tile_waves_of(nx, ny, nph, fp32 != 0); }
 int tile_blocks(int nx, int ny, int tw) { return sifv::tile_shape_of(nx, ny, tw).blocks(1); }
 int scratch_partials() { return sifv::kScratchPartials; }
+long long strip_wait_ticks(int khz) { return sifv::strip_wait_ticks(khz); }
 int stress_partials() { return sifv::kStressPartials; }
 }
 """
@@ -26,7 +28,9 @@ def shapes(tmp_path_factory):
     src, out = d / "shim.cpp", d / "shim.so"
     src.write_text(SHIM)
     subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, "-o", str(out), str(src)], check=True)
-    return C.CDLL(str(out))
+    lib = C.CDLL(str(out))
+    lib.strip_wait_ticks.restype = C.c_longlong
+    return lib
 
 
 @pytest.mark.parametrize("R", [1, 2, 3])
@@ -60,3 +64,12 @@ def test_tiles_fit_the_allocation_free_partials(shapes, nph, fp32):
         ny = 8 * (cap - stress)
         assert shapes.tile_waves(1, ny, nph, fp32) == (0 if nph and fp32 else 10)
         assert shapes.tile_waves(1, ny + 1, nph, fp32) == 0
+
+
+def test_strip_waits_are_bounded_by_time(shapes):
+    """At least 20 s, so that a sweep whose strips wait for another stream's kernels is
+    not given up, at the wall clock's 100 MHz and ten times that (more than 32 bits); a
+    rate that the device does not tell counts as 100 MHz."""
+    for khz in (100000, 1000000):
+        assert 20.0 <= shapes.strip_wait_ticks(khz) / (khz * 1e3) <= 60.0
+    assert shapes.strip_wait_ticks(0) == shapes.strip_wait_ticks(100000)
