@@ -1645,16 +1645,10 @@ int setup_igr(sifv_handle* h) {
             &perCuS, reinterpret_cast<const void*>(igr_strip_kernels().sweep), kStripWaves * kWave, 0));
         if (W <= perCuS * cus) {
             const bool perX = h->sbc[0] == BK_WRAP;
-            const int gap = perX ? std::max(0, W * kWave + kWave + 4 * kStripGroup - h->ny) : 0;
+            const StripPeriod sp = strip_period(h->ny, W, perX);
             h->igrStrips = W;
-            h->igrPeriod = h->ny + gap;
-            h->igrSlots = h->igrPeriod;
-            if (sizeof(double) * (size_t)W * h->igrSlots * kStripSlot > (size_t)2 << 30 && gap > 0) {
-                // slots for the gap rows too would cost more than 2 GiB: as many
-                // slots as rows, and a period of whole multiples of them
-                h->igrSlots = h->ny;
-                h->igrPeriod = (h->igrPeriod + h->ny - 1) / h->ny * h->ny;
-            }
+            h->igrPeriod = sp.period;
+            h->igrSlots = sp.slots;
             HIPCHK(hipMalloc(&h->igrRec, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
             HIPCHK(hipMemset(h->igrRec, 0, sizeof(double) * (size_t)W * h->igrSlots * kStripSlot));
             // tagged edge values [2][W][ny][2] per side (tag 0: none)

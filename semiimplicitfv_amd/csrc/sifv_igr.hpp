@@ -383,8 +383,8 @@ __global__ void __launch_bounds__(64) igr_sweep_kernel(IgrSweepArgs A) {
 // arrays (by sweep parity), handed over per group of kStripGroup steps.  On a
 // wrapping x axis sweep q of strip 0 needs sweep q-1 of the last strip on the same
 // row, while each strip trails its left neighbour by 64 steps and more: the gap
-// between sweeps makes room for that skew (gap = 64 W + 64 + 4 groups - ny when
-// positive, 72 steps more than the dependencies need).
+// between sweeps makes room for that skew (strip_period(): 64 W + 64 + 32 steps, 72
+// more than the dependencies need).
 // What bounds it: the serial chain of a group (8 steps of two dependent multiply-
 // adds and a shift, with the LDS reads and counters around them about 0.65 us)
 // times (ny + 64 W) / 8, and around a wrapping axis the hand-off of every strip

@@ -83,4 +83,24 @@ inline int tile_waves_of(int nx, int ny, int nph, bool fp32) {
 // of `khz` (the device's wall clock: 100 MHz, also where the rate is not told).
 constexpr long long strip_wait_ticks(int khz) { return 30LL * 1000 * (khz > 0 ? khz : 100000); }
 
+// Period of the IGR strips' sweeps (steps from one sweep to the next) and record
+// slots per strip, of which the period is a multiple.  On a wrapping x axis a sweep
+// trails its wrap neighbour by the skew of all W strips (and 32 steps of margin), so
+// a period of a mesh with fewer rows has idle rows.  They need no slots of their own:
+// the period is split into as many runs of slots as it holds ny (a remainder up to
+// ny / 16 short of one more counts as that one), so the slots stay below 2 ny and the
+// period grows by less than a run's remainder, or by ny / 16.  4096 x 152: 156 slots
+// and 4212 steps instead of 4192 of both, 31 MB of records instead of 824; slots of
+// ny rows alone would cost 1024^2 a period of 2048 steps instead of 1120.
+struct StripPeriod {
+    int period, slots;
+};
+inline StripPeriod strip_period(int ny, int W, bool perX) {
+    constexpr int lanes = 64, margin = 32;
+    const int need = perX ? std::max(ny, W * lanes + lanes + margin) : ny;
+    const int runs = (need + ny / 16) / ny;
+    const int slots = std::max(ny, (need + runs - 1) / runs);
+    return StripPeriod{runs * slots, slots};
+}
+
 }  // namespace sifv

@@ -21,6 +21,8 @@ STRIPS = {
     "last_strip_one_column_walls": ((129, 160), (0, 1, 0), 7, 2, 2),
     "period_without_idle_rows": ((70, 400), (1, 1, 0), 6, 3, 2),
     "slots_repeat_in_a_period": ((6720, 152), (1, 1, 0), 3, 2, 2),
+    "slots_of_the_rows_alone": ((704, 200), (1, 1, 0), 3, 2, 2),
+    "slots_of_some_idle_rows_walls_y": ((400, 190), (1, 0, 0), 3, 2, 2),
 }
 
 

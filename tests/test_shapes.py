@@ -1,6 +1,7 @@
 """Index and shape arithmetic of csrc/sifv_shapes.hpp, compiled here with the host
 compiler: the LDS rings of the marching kernels, the rule that picks
-stage tiles, the bound of the IGR strips' waits."""
+stage tiles, the bound of the IGR strips' waits and
+their period and record slots."""
 import ctypes as C
 import os
 import subprocess
@@ -17,6 +18,11 @@ int tile_waves(int nx, int ny, int nph, int fp32) { return sifv::tile_waves_of(n
 int tile_blocks(int nx, int ny, int tw) { return sifv::tile_shape_of(nx, ny, tw).blocks(1); }
 int scratch_partials() { return sifv::kScratchPartials; }
 long long strip_wait_ticks(int khz) { return sifv::strip_wait_ticks(khz); }
+void strip_period(int ny, int W, int perX, int* p) {
+    const sifv::StripPeriod s = sifv::strip_period(ny, W, perX != 0);
+    p[0] = s.period;
+    p[1] = s.slots;
+}
 int stress_partials() { return sifv::kStressPartials; }
 }
 """
@@ -73,3 +79,21 @@ def test_strip_waits_are_bounded_by_time(shapes):
     for khz in (100000, 1000000):
         assert 20.0 <= shapes.strip_wait_ticks(khz) / (khz * 1e3) <= 60.0
     assert shapes.strip_wait_ticks(0) == shapes.strip_wait_ticks(100000)
+
+
+def test_strip_period_and_slots(shapes):
+    """Slots for every row and for less than twice the rows, a period of whole multiples
+    of them with room for the skew of all strips, at most 1/16 and a few steps more."""
+    out = (C.c_int * 2)()
+    for ny in list(range(152, 420)) + [1000, 1024, 2048, 4097, 8192, 20000]:
+        for W in (1, 2, 3, 4, 11, 16, 64, 105, 128, 256):
+            shapes.strip_period(ny, W, 0, out)
+            assert tuple(out) == (ny, ny)
+            shapes.strip_period(ny, W, 1, out)
+            period, slots = out
+            need = max(ny, 64 * W + 96)
+            assert ny <= slots < 2 * ny and period % slots == 0
+            assert need <= period <= need + max(period // slots, ny // 16)
+    for (ny, W), want in {(1024, 16): (1120, 1120), (152, 64): (4212, 156), (200, 11): (800, 200)}.items():
+        shapes.strip_period(ny, W, 1, out)
+        assert tuple(out) == want
