@@ -64,18 +64,21 @@ inline StageShape tile_shape_of(int nx, int ny, int waves) {
 // stage, or 0 for the marching kernel.  Meshes whose marching waves cannot fill
 // the chip take tiles: a wave's serial chain of 6 rows costs 22 us there, a
 // tile 11 us (128^2 FP64; 128^2 water/air 44 -> 16 us, FP32 21 -> 10 us).  The
-// line is where the tiles' halo rows and barriers cost more than that:
-// 576^2 30.4 against 34.9 us and 640^2 36.8 against 35.4 (FP64), 768^2 28.6
-// against 31.7 and 896^2 37.6 against 36.7 (FP32), 800^2 99 against 102
-// (water/air).  Small tiles (2 rows) while those of 8 rows would leave half
-// the 256 CUs idle: 128^2 10.8 against 12.8 us, 320^2 16.0 against 13.7.
-// A mesh of few columns whose tiles are more than the allocation-free loop has
-// dt partials for marches (1 x 600000 water/air: 75000 tiles).
+// line is where the 256 CUs take one more round of tiles than that is worth, and
+// lies in tiles, not in cells: a strip of 8 columns costs what one of 62 does.
+// us a step of 3 stages, tiles against march, with the number of 8-row tiles:
+//   FP64       752: 83 / 97 (190x1500),  720: 83 / 97 (576^2),  810: 98 / 97
+//              (5000x80),  880: 104 / 98 (640^2),  2500: 249 / 178 (8x20000)
+//   FP32       1222: 76 / 89 (750^2),  1300: 89 / 90 (800^2),  2500: 160 / 124
+//   water/air  1222: 232 / 267 (750^2),  1250: 234 / 264 (63x5000),  1300: 274 / 271
+//              and with LF 284 / 273 (800^2),  2125: 406 / 375 (1000^2),  2500: 453 /
+//              400; below it 880: 187 / 182 (640^2) and 1000: 190 / 182 (80x4000) lose
+// Small tiles (2 rows) while those of 8 rows would leave half the 256 CUs idle:
+// 128^2 10.8 against 12.8 us a stage, 320^2 16.0 against 13.7.
 inline int tile_waves_of(int nx, int ny, int nph, bool fp32) {
     if (fp32 && nph) return 0;
-    if ((long)nx * ny > (nph ? 640000 : fp32 ? 600000 : 360000)) return 0;
     const int blocks = tile_shape_of(nx, ny, kTileWaves).blocks(1);
-    if (blocks > kScratchPartials - kStressPartials) return 0;
+    if (blocks > (fp32 || nph ? 1280 : 768)) return 0;
     return blocks < 128 ? kTileSmall : kTileWaves;
 }
 

@@ -65,11 +65,12 @@ def test_tiles_fit_the_allocation_free_partials(shapes, nph, fp32):
                 tiled += 1
                 assert shapes.tile_blocks(nx, ny, tw) + stress <= cap, (nx, ny)
     assert (tiled == 0) == bool(nph and fp32)
-    # as many 8-row tiles as there is room for beside the stress limits, and one more
-    if nph or fp32:
-        ny = 8 * (cap - stress)
-        assert shapes.tile_waves(1, ny, nph, fp32) == (0 if nph and fp32 else 10)
-        assert shapes.tile_waves(1, ny + 1, nph, fp32) == 0
+    # the line is in tiles of 62 columns x 8 rows: full strips and strips of 8 columns alike
+    line = 0 if nph and fp32 else 1280 if nph or fp32 else 768
+    for nx, strips in ((8, 1), (62, 1), (63, 2), (496, 8)):
+        ny = 8 * (line // strips)
+        assert shapes.tile_waves(nx, max(ny, 1), nph, fp32) == (10 if line else 0)
+        assert shapes.tile_waves(nx, ny + 8, nph, fp32) == 0
 
 
 def test_strip_waits_are_bounded_by_time(shapes):

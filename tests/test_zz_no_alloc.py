@@ -121,8 +121,8 @@ def test_noalloc_refusals(gpu):
 
 @pytest.mark.parametrize("precision,two", [("fp64", True), ("mixed", False)])
 def test_noalloc_one_column(gpu, precision, two):
-    """600000 rows of one column: on 8-row tiles they would need 75000 dt partials,
-    more than the static array holds; the march they take needs 18750."""
+    """600000 rows of one column: 75000 dt partials on 8-row tiles, more than the static
+    array holds; 18750 as the march that they take."""
     def build():
         if two:
             cfg, mesh, st, eos = make_two_phase_case(2, (1, 600000), seed=9, p_jump=False)
