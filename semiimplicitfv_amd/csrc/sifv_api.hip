@@ -1293,7 +1293,7 @@ struct MgCycle {
         if (!r)
             r = launch(by_dim(dim, mg_restrict_fine_kernel<1, R>, mg_restrict_fine_kernel<2, R>,
                               mg_restrict_fine_kernel<3, R>),
-                       dim >= 2 && sizeof(R) == 8 ? nb : cgrid(M.C.cells));
+                       dim == 3 && sizeof(R) == 8 ? nb : cgrid(M.C.cells));
         // levels m..L-1 (at most SIFV_MG_TAIL_CELLS cells each) run in one
         // workgroup, the coarsest included
         int m = L - 1;

@@ -23,7 +23,7 @@
 // the slot one past the last cell of a line holds the line's high boundary
 // face (0 on a wall, the wrap face of a periodic axis), so a row reads its
 // high weight from the next slot.  The set-up, the coarse operators, the FP32
-// V-cycle and 1D read them; in 2D/3D the passes over the fine level form the
+// V-cycle, 1D and 2D read them; in 3D the passes over the fine level form the
 // weights again from rho (RhoRow), which is less to read.  Scalars
 // (alpha, beta, the dot products) stay on the device; each product and update
 // kernel writes per-block partial sums that a one-block kernel folds in fixed
@@ -31,9 +31,9 @@
 // iteration: the host enqueues iterations in chunks and polls the flag.
 //
 // Per iteration, per interior cell: pcg_matvec (read p with its 2*DIM
-// neighbours, rho, s; write q: 32 B in 2D/3D), pcg_update (read x p r q d s,
-// write x r z: 72 B), pcg_dir (read z p, write p: 24 B) -- 128 B/cell,
-// HBM-bound.
+// neighbours, rho in 3D or the weights, s; write q: 32 B in 3D, 40 in 2D),
+// pcg_update (read x p r q d s, write x r z: 72 B), pcg_dir (read z p, write p:
+// 24 B) -- 128 B/cell in 3D, HBM-bound.
 #pragma once
 
 #include "sifv_aux.hpp"
@@ -203,7 +203,15 @@ __device__ __forceinline__ void pcg_columns(const Grid& g, F&& body) {
     }
 }
 
-// A row of S in a column (i, j) of a 2D/3D mesh with the face weights formed from the
+template <int DIM, typename F>
+__device__ __forceinline__ void pcg_bricks(const Grid& g, F&& body) {
+    pcg_columns<DIM, 1>(g, [&](int i, int j, int k0, int k1) __attribute__((always_inline)) {
+        if (i >= g.nx || j >= g.ny) return;
+        for (int k = k0; k < k1; ++k) body(i, j, k);
+    });
+}
+
+// A row of S in a column (i, j) of a 3D mesh with the face weights formed from the
 // densities: w = 4 area / ((rho + rho_nb)(h + h_nb)), the two faces of a direction
 // from one reciprocal.  The passes over the fine level are bound by memory, so 8 B of
 // rho instead of 24 B of weights (and instead of the diagonal's 8, where both are
@@ -211,8 +219,9 @@ __device__ __forceinline__ void pcg_columns(const Grid& g, F&& body) {
 // kept over its planes, and density and v are carried from plane to plane.  A wall's
 // weight is 0 and its neighbour the cell itself.  At 256^3, from stored weights -> from
 // densities -> carried up the column: product 138 -> 140 -> 120 us, restriction
-// 174 -> 150 -> 135, post-smoothing 193 -> 186 -> 159.
-template <int DIM>
+// 174 -> 150 -> 135, post-smoothing 193 -> 186 -> 159.  In 2D there are no planes to
+// carry anything up and 16 B of weights to save 8 of, and it was slower (a PCG step of
+// 1500x1024 20.9 -> 23.6 ms, multigrid PCG 24.5 -> 26.7): 2D reads the weights.
 struct RhoRow {
     double gxl, gxr, gyl, gyr, hxy;
     int pxl, pxr, pyl, pyr;   // offsets of the neighbours (wrapped)
@@ -248,12 +257,10 @@ struct RhoRow {
         const size_t id = cell_index(g, i, j, k);
         rm = rc = A.rho[id];
         vm = vc = val(id, i, j, k);
-        if (DIM >= 3) {
-            const long sz = (long)g.nxT * g.nyT;
-            const int kl = pcg_nbc(g, 2, 0, k);
-            if (k > 0 || g.sbc[4] == BK_WRAP) rm = A.rho[id - sz];
-            vm = val(id + (kl - k) * sz, i, j, kl);
-        }
+        const long sz = (long)g.nxT * g.nyT;
+        const int kl = pcg_nbc(g, 2, 0, k);
+        if (k > 0 || g.sbc[4] == BK_WRAP) rm = A.rho[id - sz];
+        vm = val(id + (kl - k) * sz, i, j, kl);
     }
     // (S v) at the next plane k; vi: v there; dd: the diagonal
     template <typename V>
@@ -263,30 +270,22 @@ struct RhoRow {
         const double* __restrict__ rho = A.rho;
         double sxl = rc + rho[id + rxl], sxr = rc + rho[id + rxr];
         double syl = rc + rho[id + ryl], syr = rc + rho[id + ryr];
-        double szl = 1.0, szr = 1.0, nzl = 0.0, nzr = 0.0, hl = 1.0, hr = 1.0;
         vi = vc;
         const double vxl = val(id + pxl, il, j, k), vxr = val(id + pxr, ir, j, k);
         const double vyl = val(id + pyl, i, jl, k), vyr = val(id + pyr, i, jr, k);
-        double vzr = 0.0, rp = 0.0;
         const double vzl = vm;
         const double hz = g.dzw[k + g.ngz];
-        if (DIM >= 3) {
-            const long sz = (long)g.nxT * g.nyT;
-            const int kr = pcg_nbc(g, 2, 1, k);
-            const bool wl = k == 0 && g.sbc[4] != BK_WRAP, wr = k == g.nz - 1 && g.sbc[5] != BK_WRAP;
-            rp = rho[id + (wr ? 0 : sz)];
-            szl = rc + rm;
-            szr = rc + rp;
-            nzl = wl ? 0.0 : hxy;
-            nzr = wr ? 0.0 : hxy;
-            hl = g.dzw[k - 1 + g.ngz] + hz;
-            hr = hz + g.dzw[k + 1 + g.ngz];
-            vzr = val(id + (kr - k) * sz, i, j, kr);
-        }
+        const long sz = (long)g.nxT * g.nyT;
+        const int kr = pcg_nbc(g, 2, 1, k);
+        const bool wl = k == 0 && g.sbc[4] != BK_WRAP, wr = k == g.nz - 1 && g.sbc[5] != BK_WRAP;
+        const double rp = rho[id + (wr ? 0 : sz)];
+        double szl = rc + rm, szr = rc + rp;
+        const double nzl = wl ? 0.0 : hxy, nzr = wr ? 0.0 : hxy;
+        const double hl = g.dzw[k - 1 + g.ngz] + hz, hr = hz + g.dzw[k + 1 + g.ngz];
+        const double vzr = val(id + (kr - k) * sz, i, j, kr);
         // densities under the floor are rare: look once for all faces (a NaN is under
         // nothing, and stays)
-        double lo = fmin(fmin(sxl, sxr), fmin(syl, syr));
-        if (DIM >= 3) lo = fmin(lo, fmin(szl, szr));
+        const double lo = fmin(fmin(fmin(sxl, sxr), fmin(syl, syr)), fmin(szl, szr));
         if (__builtin_expect(lo < 2e-14, 0)) {
             sxl = dmax_ref(sxl, 2e-14);
             sxr = dmax_ref(sxr, 2e-14);
@@ -307,7 +306,7 @@ struct RhoRow {
         };
         faces(sxl, sxr, gxl * hz, gxr * hz, vxl, vxr);
         faces(syl, syr, gyl * hz, gyr * hz, vyl, vyr);
-        if (DIM >= 3) faces(szl * hl, szr * hr, nzl, nzr, vzl, vzr);
+        faces(szl * hl, szr * hr, nzl, nzr, vzl, vzr);
         // an infinite density, or a product of two faces out of range, leaves a NaN:
         // one reciprocal per face, 0 for an infinite density
         if (__builtin_expect(!(dd >= 0.0), 0)) {
@@ -322,10 +321,8 @@ struct RhoRow {
             face(sxr, gxr * hz, vxr);
             face(syl, gyl * hz, vyl);
             face(syr, gyr * hz, vyr);
-            if (DIM >= 3) {
-                face(szl * hl, nzl, vzl);
-                face(szr * hr, nzr, vzr);
-            }
+            face(szl * hl, nzl, vzl);
+            face(szr * hr, nzr, vzr);
         }
         rm = rc;
         rc = rp;
@@ -463,12 +460,12 @@ __global__ void __launch_bounds__(256) pcg_matvec_kernel(PcgArgs A) {
     __shared__ double sh[256 / kWave];
     const Grid& g = A.g;
     double pq = 0.0;
-    if constexpr (DIM >= 2) {
+    if constexpr (DIM == 3) {
         const double* __restrict__ p = A.p;
         auto val = [&](size_t n, int, int, int) __attribute__((always_inline)) { return p[n]; };
         pcg_columns<DIM, 1>(g, [&](int i, int j, int k0, int k1) {
             if (i >= g.nx || j >= g.ny) return;
-            RhoRow<DIM> R(g, i, j);
+            RhoRow R(g, i, j);
             R.begin(A, val, i, j, k0);
             for (int k = k0; k < k1; ++k) {
                 const size_t id = cell_index(g, i, j, k);
@@ -479,12 +476,17 @@ __global__ void __launch_bounds__(256) pcg_matvec_kernel(PcgArgs A) {
             }
         });
     } else {
-        int i, j, k;
-        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) {
+        auto cell = [&](int i, int j, int k) __attribute__((always_inline)) {
             const size_t id = cell_index(g, i, j, k);
             const double qv = pcg_row<DIM>(A, A.p, A.s[id], i, j, k, id);
             A.q[id] = qv;
             pq += A.p[id] * qv;
+        };
+        if constexpr (DIM == 2) {
+            pcg_bricks<DIM>(g, cell);
+        } else {
+            int i, j, k;
+            for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k);
         }
     }
     pcg_partials(A, sh, 1, pq, 0.0, 0.0);
@@ -593,8 +595,9 @@ __global__ void __launch_bounds__(256) pcg_dir_kernel(PcgArgs A) {
 // is a fixed SPD operator and conjugate gradients stay valid.
 // Fine-level work per V-cycle and cell: pre (q = om r / d, folded into
 // pcg_update_kernel inside the iteration), restrict (read q and rho with
-// neighbours, s, r: 32 B in 2D/3D), prolong and post in one pass (read q rho s r
-// and the parent's correction, write z, with the r.z partial sums: 40 B).
+// neighbours, s, r: 32 B in 3D; the weights for rho in 2D), prolong and post in one
+// pass (read q rho s r and the parent's correction, write z, with the r.z partial
+// sums: 40 B).
 constexpr int kMgMaxLevels = 24;
 constexpr int kMgCoarseSweeps = 16;
 
@@ -762,7 +765,7 @@ __global__ void __launch_bounds__(256) mg_restrict_fine_kernel(MgArgsT<R> M) {
     const PcgArgs& A = M.A;
     const Grid& g = A.g;
     const MgLevelT<R>& C = M.C;
-    if constexpr (DIM >= 2 && sizeof(R) == 8) {
+    if constexpr (DIM == 3 && sizeof(R) == 8) {
         // a thread sums the children of its column in two rows and two planes, its
         // neighbour lane adds the other column's
         const double* __restrict__ q = A.q;
@@ -770,7 +773,7 @@ __global__ void __launch_bounds__(256) mg_restrict_fine_kernel(MgArgsT<R> M) {
         pcg_columns<DIM, 2>(g, [&](int i, int j, int k0, int k1) {
             const bool on = i < g.nx && j < g.ny;
             const int ic = min(i, g.nx - 1), ja = min(j, g.ny - 1), jb = min(j + 1, g.ny - 1);
-            RhoRow<DIM> Ra(g, ic, ja), Rb(g, ic, jb);
+            RhoRow Ra(g, ic, ja), Rb(g, ic, jb);
             Ra.begin(A, val, ic, ja, k0);
             Rb.begin(A, val, ic, jb, k0);
             for (int k = k0; k < k1; k += 2) {
@@ -825,47 +828,57 @@ __global__ void __launch_bounds__(256) mg_post_fine_kernel(MgArgsT<R> M) {
     constexpr double om = mg_omega(DIM);
     const R* __restrict__ tc = C.t;
     double rz = 0.0;
-    const double* __restrict__ q64 = A.q;
-    auto qp64 = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
-        return q64[n] + (double)tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
-    };
-    auto cell = [&](int i, int j, int k, RhoRow<DIM>* R2) __attribute__((always_inline)) {
-        const size_t id = cell_index(g, i, j, k);
-        const double r = A.r[id];
-        double z;
-        if constexpr (sizeof(R) == 4) {
-            const float* __restrict__ q = M.f32.q;
-            auto qp = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
-                return q[n] + tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
-            };
-            float qi;
-            const float a = face_row<DIM, float>(g, M.f32.W, qp, M.f32.s[id], i, j, k, id, qi);
-            z = (double)(qi + (float)om * ((float)r - a) / M.f32.d[id]);
-        } else {
-            double qi, dd;
-            double a;
-            if constexpr (DIM >= 2) {
-                a = R2->row(A, qp64, A.s[id], i, j, k, id, qi, dd);
-            } else {
-                a = pcg_row_f<DIM>(A, qp64, A.s[id], i, j, k, id, qi);
-                dd = A.d[id];
-            }
-            z = qi + om * (r - a) / dd;
-        }
+    // z from (S q', q', d) of a cell
+    auto put = [&](size_t id, double r, double a, double qi, double dd) __attribute__((always_inline)) {
+        const double z = qi + om * (r - a) / dd;
         A.z[id] = z;
         rz += r * z;
         if (M.init) A.p[id] = z;
     };
-    if constexpr (DIM >= 2) {
+    const double* __restrict__ q64 = A.q;
+    auto qp64 = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
+        return q64[n] + (double)tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
+    };
+    if constexpr (DIM == 3 && sizeof(R) == 8) {
         pcg_columns<DIM, 1>(g, [&](int i, int j, int k0, int k1) {
             if (i >= g.nx || j >= g.ny) return;
-            RhoRow<DIM> R2(g, i, j);
-            if constexpr (sizeof(R) == 8) R2.begin(A, qp64, i, j, k0);
-            for (int k = k0; k < k1; ++k) cell(i, j, k, &R2);
+            RhoRow R2(g, i, j);
+            R2.begin(A, qp64, i, j, k0);
+            for (int k = k0; k < k1; ++k) {
+                const size_t id = cell_index(g, i, j, k);
+                const double r = A.r[id];
+                double qi, dd;
+                const double a = R2.row(A, qp64, A.s[id], i, j, k, id, qi, dd);
+                put(id, r, a, qi, dd);
+            }
         });
     } else {
-        int i, j, k;
-        for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k, nullptr);
+        auto cell = [&](int i, int j, int k) __attribute__((always_inline)) {
+            const size_t id = cell_index(g, i, j, k);
+            const double r = A.r[id];
+            if constexpr (sizeof(R) == 4) {
+                const float* __restrict__ q = M.f32.q;
+                auto qp = [&](size_t n, int a, int b, int c) __attribute__((always_inline)) {
+                    return q[n] + tc[mg_idx(C, a >> 1, b >> 1, c >> 1)];
+                };
+                float qi;
+                const float a = face_row<DIM, float>(g, M.f32.W, qp, M.f32.s[id], i, j, k, id, qi);
+                const double z = (double)(qi + (float)om * ((float)r - a) / M.f32.d[id]);
+                A.z[id] = z;
+                rz += r * z;
+                if (M.init) A.p[id] = z;
+            } else {
+                double qi;
+                const double a = pcg_row_f<DIM>(A, qp64, A.s[id], i, j, k, id, qi);
+                put(id, r, a, qi, A.d[id]);
+            }
+        };
+        if constexpr (DIM >= 2) {
+            pcg_bricks<DIM>(g, cell);
+        } else {
+            int i, j, k;
+            for (InteriorIter it_(g.nx, g.ny, g.nz); it_.next(i, j, k);) cell(i, j, k);
+        }
     }
     const double t = wave_sum(rz);
     const int w = threadIdx.x / kWave, l = threadIdx.x % kWave;
