@@ -177,11 +177,11 @@ __device__ __forceinline__ double pcg_row_f(const PcgArgs& A, V&& val, double si
 constexpr int kBrickPlanes = 16;
 
 template <int DIM, int RY, typename F>
-__device__ __forceinline__ void pcg_columns(const Grid& g, F&& body) {
+__device__ __forceinline__ void pcg_columns(const Grid& g, F&& body, int planes = kBrickPlanes) {
     // body(i, j, k0, k1): column i of rows j .. j + RY - 1, also past the mesh's edges
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
     const int bx = (g.nx + 63) / 64, by = (g.ny + 4 * RY - 1) / (4 * RY);
-    const int bz = DIM == 3 ? (g.nz + kBrickPlanes - 1) / kBrickPlanes : 1;
+    const int bz = DIM == 3 ? (g.nz + planes - 1) / planes : 1;
     const long nbr = (long)bx * by * bz;
     const int G = (int)gridDim.x;
     long lo = 0, hi = nbr, t0 = blockIdx.x, step = G;
@@ -197,8 +197,8 @@ __device__ __forceinline__ void pcg_columns(const Grid& g, F&& body) {
         const int cy = (int)(t % by);
         const long rest = t / by;
         const int cx = (int)(rest % bx), cz = (int)(rest / bx);
-        const int k0 = DIM == 3 ? cz * kBrickPlanes : 0;
-        const int k1 = DIM == 3 ? min(g.nz, k0 + kBrickPlanes) : 1;
+        const int k0 = DIM == 3 ? cz * planes : 0;
+        const int k1 = DIM == 3 ? min(g.nz, k0 + planes) : 1;
         body(cx * 64 + tx, (cy * 4 + ty) * RY, k0, k1);
     }
 }
@@ -789,7 +789,7 @@ __global__ void __launch_bounds__(256) mg_restrict_fine_kernel(MgArgsT<R> M) {
                 if (i + 1 < g.nx) acc += other;
                 if (on && (i & 1) == 0) C.b[mg_idx(C, i >> 1, j >> 1, k >> 1)] = acc;
             }
-        });
+        }, restrict_planes(g.nx, g.ny, g.nz));
         return;
     }
     const float* __restrict__ q32 = M.f32.q;

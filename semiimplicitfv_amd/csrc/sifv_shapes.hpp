@@ -82,6 +82,23 @@ inline int tile_waves_of(int nx, int ny, int nph, bool fp32) {
     return blocks < 128 ? kTileSmall : kTileWaves;
 }
 
+// Planes a thread of the multigrid's fine restriction walks (3D, FP64; a brick is 64
+// columns x 8 rows): up to 16, to carry densities and vector up the column, as long as
+// there are 600 bricks for the 256 CUs, and never less than the 2 of a coarse cell.
+// us a launch with 2 / 4 / 8 / 16 planes, and of the form before the walk:
+//   24^3            4.8 /   6.4 /   9.5 /  15.1,   5.3
+//   48x64x40        5.4 /   7.3 /  10.5 /  16.9,   5.6
+//   90x80x70        7.4 /   8.1 /   9.8 /  15.6,   5.7
+//   128x100x96     12.4 /  11.9 /  13.7 /  18.3,  14.1
+//   160x144x176    43.5 /  37.5 /  33.6 /  36.8,  53.8
+//   224^3         158   / 135   / 125   / 127,    162
+constexpr int restrict_planes(int nx, int ny, int nz) {
+    const long columns = (long)((nx + 63) / 64) * ((ny + 7) / 8);
+    int p = 16;
+    while (p > 2 && columns * ((nz + p - 1) / p) < 600) p /= 2;
+    return p;
+}
+
 // Longest wait of a strip of the IGR sweep for another one, 30 s, in ticks of a clock
 // of `khz` (the device's wall clock: 100 MHz, also where the rate is not told).
 constexpr long long strip_wait_ticks(int khz) { return 30LL * 1000 * (khz > 0 ? khz : 100000); }

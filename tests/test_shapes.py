@@ -1,7 +1,7 @@
 """Index and shape arithmetic of csrc/sifv_shapes.hpp, compiled here with the host
 compiler: the LDS rings of the marching kernels, the rule that picks
 stage tiles, the bound of the IGR strips' waits and
-their period and record slots."""
+their period and record slots, the planes a thread of the fine restriction walks."""
 import ctypes as C
 import os
 import subprocess
@@ -23,6 +23,7 @@ void strip_period(int ny, int W, int perX, int* p) {
     p[0] = s.period;
     p[1] = s.slots;
 }
+int restrict_planes(int nx, int ny, int nz) { return sifv::restrict_planes(nx, ny, nz); }
 int stress_partials() { return sifv::kStressPartials; }
 }
 """
@@ -98,3 +99,10 @@ def test_strip_period_and_slots(shapes):
     for (ny, W), want in {(1024, 16): (1120, 1120), (152, 64): (4212, 156), (200, 11): (800, 200)}.items():
         shapes.strip_period(ny, W, 1, out)
         assert tuple(out) == want
+
+
+def test_restriction_walk(shapes):
+    """Whole coarse cells, and no long walks while the mesh has few columns."""
+    for n, want in {(24, 24, 24): 2, (48, 64, 40): 2, (90, 80, 70): 2, (128, 100, 96): 4, (160, 144, 176): 8,
+                    (224, 224, 224): 16, (256, 256, 256): 16, (5, 3, 2): 2, (2000, 2000, 1): 16}.items():
+        assert shapes.restrict_planes(*n) == want, n
