@@ -873,21 +873,27 @@ stage_xy_kernel(StageParams<T> P) {
     };
     // primitive rows r and r-1 (by parity) of the march: the x stencil of row r
     // and the two oldest rows of the y stencil of row r+1 (own column); sar:
-    // partial densities of row r
-    __shared__ C sp[2][NPV][kWave + 2 * E];
-    __shared__ C sar[NPH > 0 ? NPH : 1][NPH > 0 ? kWave : 1];
+    // partial densities of row r.  The two-phase 2D forms run two waves per SIMD
+    // either way and keep their own cell of row r in registers: with it in LDS they
+    // were slower than with all rows in registers (2500x2000 FP32 1288 against 1238 us
+    // a step, now 1244; upwind 3 1212 against 1186, now 1202).
+    constexpr bool CURREG = DIM == 2 && NPH > 0;
+    using S = typename std::conditional<CURREG, T, C>::type;
+    __shared__ S sp[2][NPV][kWave + 2 * E];
+    __shared__ C sar[NPH > 0 && !CURREG ? NPH : 1][NPH > 0 && !CURREG ? kWave : 1];
+    Cell<DIM, NPH, C> cur;
     // rows r+1 .. r+R, one per register slot
     Cell<DIM, NPH, C> win[R];
     T sigwin[R];
     auto putRow = [&](const Cell<DIM, NPH, C>& c, T sg, int row, int pos) __attribute__((always_inline)) {
-        C* o = &sp[row & 1][0][pos];
-        o[0] = c.rho;
+        S* o = &sp[row & 1][0][pos];
+        o[0] = (S)c.rho;
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) o[(1 + d) * (kWave + 2 * E)] = c.u[d];
-        o[(DIM + 1) * (kWave + 2 * E)] = c.p;
+        for (int d = 0; d < DIM; ++d) o[(1 + d) * (kWave + 2 * E)] = (S)c.u[d];
+        o[(DIM + 1) * (kWave + 2 * E)] = (S)c.p;
 #pragma unroll
-        for (int ph = 0; ph < NPH; ++ph) o[(DIM + 2 + ph) * (kWave + 2 * E)] = c.a[ph];
-        if constexpr (kSig) o[NV * (kWave + 2 * E)] = (C)sg;
+        for (int ph = 0; ph < NPH; ++ph) o[(DIM + 2 + ph) * (kWave + 2 * E)] = (S)c.a[ph];
+        if constexpr (kSig) o[NV * (kWave + 2 * E)] = (S)sg;
     };
     auto sigAt = [&](int c, int row) { return useSig ? (T)load_sigma<DIM>(P, c, row, kz) : T(0); };
     FaceState<DIM, NPH, T> plusPrev;
@@ -906,6 +912,7 @@ stage_xy_kernel(StageParams<T> P) {
             const T sg = sigAt(col, rStart + m);
             if (m <= 0) {
                 putRow(c, sg, rStart + m, lane + E);
+                if (CURREG && m == 0) win[0] = c;
             } else {
                 win[m] = c;
                 sigwin[m] = sg;
@@ -941,8 +948,8 @@ stage_xy_kernel(StageParams<T> P) {
 #pragma unroll
         for (int q = 0; q < NF; ++q) Ghi[q] = T(0);
         double cy = 0.0, dyr = 1.0;
-        Cell<DIM, NPH, C> cur;
         if (YDIR) {
+            if constexpr (CURREG) cur = win[0];
 #pragma unroll
             for (int m = 0; m < R - 1; ++m) {
                 win[m] = win[m + 1];
@@ -964,12 +971,14 @@ stage_xy_kernel(StageParams<T> P) {
             // y reconstruction of row r+1: rows r+2-R .. r+R, up to row r in LDS
             FaceState<DIM, NPH, T> mY, pY;
             {
-                T mn[NV], pl[NV], vv[R][NV];
+                T mn[NV], pl[NV], vv[R][NV], vc[NV];
 #pragma unroll
                 for (int m = 0; m < R; ++m) recon_vars<DIM, NPH, T>(win[m], vv[m]);
+                if constexpr (CURREG) recon_vars<DIM, NPH, T>(cur, vc);
                 recon_set<R, T, NV>(
                     [&](int v, int s) __attribute__((always_inline)) {
                         const int rel = 2 - R + s;
+                        if (CURREG && rel == 0) return vc[v];
                         return rel <= 0 ? (T)sp[(r + rel) & 1][v][lane + E] : vv[rel > 0 ? rel - 1 : 0][v];
                     },
                     eps, weno, mn, pl);
@@ -989,7 +998,11 @@ stage_xy_kernel(StageParams<T> P) {
                 riemann<RS, 1, DIM, NPH, T>(plusPrev, mY, incP, igr, F);
                 // cells of face r+1/2: rows r (LDS) and r+1
                 C rhoL = C(0), arL[NPH > 0 ? NPH : 1];
-                if constexpr (NPH > 0) {
+                if constexpr (CURREG) {
+                    rhoL = cur.rho;
+#pragma unroll
+                    for (int ph = 0; ph < NPH; ++ph) arL[ph] = cur.ar[ph];
+                } else if constexpr (NPH > 0) {
                     rhoL = sp[r & 1][0][lane + E];
 #pragma unroll
                     for (int ph = 0; ph < NPH; ++ph) arL[ph] = sar[ph][lane];
@@ -1002,7 +1015,7 @@ stage_xy_kernel(StageParams<T> P) {
 #pragma unroll
                 for (int q = 0; q < NF; ++q) Glo[q] = Ghi[q];
                 putRow(win[0], sigwin[0], r + 1, lane + E);
-                if constexpr (NPH > 0) {
+                if constexpr (NPH > 0 && !CURREG) {
 #pragma unroll
                     for (int ph = 0; ph < NPH; ++ph) sar[ph][lane] = win[0].ar[ph];
                 }
@@ -1033,7 +1046,7 @@ stage_xy_kernel(StageParams<T> P) {
             putRow(ce, sigAt(ecol, r), r, lane < E ? lane : kWave + lane);
         }
         __syncthreads();
-        if (YDIR) {
+        if constexpr (YDIR && !CURREG) {
             const C* o = &sp[r & 1][0][lane + E];
             cur.rho = o[0];
 #pragma unroll
@@ -1129,7 +1142,7 @@ stage_xy_kernel(StageParams<T> P) {
             for (int q = 0; q < NF; ++q) Glo[q] = Ghi[q];
             // row r+1 takes row r-1's place
             putRow(win[0], sigwin[0], r + 1, lane + E);
-            if constexpr (NPH > 0) {
+            if constexpr (NPH > 0 && !CURREG) {
 #pragma unroll
                 for (int ph = 0; ph < NPH; ++ph) sar[ph][lane] = win[0].ar[ph];
             }
