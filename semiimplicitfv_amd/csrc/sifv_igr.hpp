@@ -533,14 +533,20 @@ __device__ __forceinline__ double dpp_shl1_in(double v, double edge) {
 //   wave 4 publishes the edge values of the groups wave 0 finishes;
 //   waves 5 and 6 poll the left and the right neighbour's edge values of upcoming
 //     groups, up to kStripRing steps ahead.
-// A record is loaded again no earlier than P - 8 (kStripRecGroups + 4) steps after
-// the step that stored its sigma; wave 0 has at most seven groups of stores
-// outstanding when it counts a group as done, so that store is complete for every
-// P >= 129 (waiting for all but two groups made the stores' latency the limit).
+// The sigma that wave 0 stores into a record is read again P steps later (slots that
+// come round sooner belong to idle rows, whose values nothing uses).  That record is
+// loaded at most kStripRecGroups + 4 groups ahead of the groups counted as done, and
+// wave 0 counts a group as done with the stores of at most kStripStoreGroups groups
+// outstanding (waiting for all but two groups made the stores' latency the limit), so
+// the store is complete if the steps of a period that store anything, ny or more and
+// so at least kStripMinRows, exceed all of them together.
 // Every wait is bounded, by time (strips may wait for CUs that another stream's
 // kernels hold, and a pass of a wave that polls LDS is some 50 ns), and ends on the
 // abort flag.
 constexpr int kStripRecGroups = 5;
+constexpr int kStripStoreGroups = 7;
+static_assert(kStripMinRows > kStripGroup * (kStripRecGroups + 4 + kStripStoreGroups), "a store before its reload");
+static_assert(kStripGroup * kStripStoreGroups <= 63, "the counter of vector memory operations has 6 bits");
 constexpr int kStripWaves = 7;
 constexpr int kStripRing = 192;   // steps of wave 0's results and inputs held in LDS
 
@@ -890,7 +896,8 @@ __global__ void __launch_bounds__(64 * kStripWaves) igr_strip_kernel(IgrStripArg
                 if (++tc == ns) tc = 0;
             }
         }
-        asm volatile("s_waitcnt vmcnt(56)" ::: "memory");   // stores of all but seven groups are done
+        // stores of all but the last kStripStoreGroups groups are done
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kStripGroup * kStripStoreGroups) : "memory");
         lds_store(&sFlag[4], g + 1);
         count(l, d, p);
         if ((pos += U) >= P) pos -= P;
