@@ -7,7 +7,7 @@ import pytest
 
 from semiimplicitfv_amd import HLLCSolver, IdealGasEOS, JacobiPressureSolver, SemiImplicitSolver
 from tests.golden import problems
-from tests.helpers import rel_errs
+from tests.helpers import make_semi_case, rel_errs
 from tests.test_gpu_semi import _tile_problem
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +52,25 @@ def test_jacobi_infinite_density(gpu, oracle_c, shape):
     l1, li = rel_errs(mesh.interior(pg), mesh.interior(pc))
     assert l1 <= 2e-14 and li <= 2e-14, (l1, li)
     g.close()
+
+
+@pytest.mark.parametrize("shape", [(63, 4, 3), (64, 3, 4), (5, 9, 7), (65, 4, 21), (67, 6)])
+def test_mixed_jacobi_planes_in_flight(gpu, shape):
+    """The FP32 correction sweeps and the FP64 passes take the same pipeline as the FP64
+    sweeps: a mixed-precision step, past its FP64 opening chunk of 4 sweeps, against the
+    FP64 solver's, to the 1e-8 of the solves' tolerance (test_mixed_precision_jacobi)."""
+    periods = (0, 1, 1) if shape[-1] % 2 else (1, 0, 0)
+    out = []
+    for precision in ("fp64", "mixed"):
+        cfg, mesh, st, eos = make_semi_case(len(shape), shape, periods=periods[:len(shape)] + (0,) * (3 - len(shape)),
+                                            seed=sum(shape), tol=1e-9, maxit=2000)
+        g = SemiImplicitSolver(mesh, HLLCSolver(eos), JacobiPressureSolver(), eos, None, cfg, precision=precision)
+        g.upload(st)
+        for k in range(2):
+            cfg.step = k
+            g.step_resident(cfg)
+            assert 4 < g.lastPressureIterations() < 2000
+        out.append([mesh.interior(g.download_field(f)).copy() for f in st.field_ids()])
+        g.close()
+    for a, b in zip(*out):
+        assert rel_errs(b, a)[0] <= 1e-8

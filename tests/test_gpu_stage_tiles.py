@@ -71,6 +71,86 @@ def test_tile_matches_march(gpu, n, kind, rs, per, precision):
             assert abs(a[f]).max() == 0.0
 
 
+def _build_more(n, kind, per, precision):
+    """The forms above with sources, a stiffened gas (pressure 1..4 beside 6e3) and, in
+    FP32, without the jump."""
+    periods = (1, 1, 0) if per else (0, 0, 0)
+    if kind == "two_source":
+        cfg, mesh, st, eos = problems.make_two_phase_case(2, n, bcs=WALLS, periods=periods, seed=64, p_jump=False)
+        cfg.viscousParams.phaseMu = [5.0, 0.5]
+        cfg.surfaceTensionParams.sigma = 1e3
+    else:
+        cfg, mesh, st, eos = problems.make_case(2, n, bcs=WALLS, periods=periods, seed=65, cfl=0.4,
+                                                nonuniform=kind == "stretched", shock=precision == "fp64",
+                                                eos_kind="stiff" if kind == "stiff" else "ideal")
+        if kind == "source":
+            cfg.viscousParams.mu = 1e-3
+        if kind == "igr":
+            cfg.useIGR = True
+            cfg.igrParams.IGRIters, cfg.igrParams.IGRWarmStartIters = 2, 3
+    if kind in ("source", "two_source"):
+        cfg.bodyForceParams.a = [0.1, -0.5, 0.0]
+    return cfg, mesh, st, eos
+
+
+MORE = [(n, k, rs, per, "mixed") for n in SMALL[1:] + LARGE
+        for k, rs, per in (("plain", 0, False), ("stretched", 1, False), ("source", 2, True), ("igr", 0, True))]
+MORE += [(n, k, rs, per, p) for n in [(62, 8), (63, 9)] + LARGE
+         for k, rs, per, p in (("two_source", 2, False, "fp64"), ("two_source", 0, True, "fp64"),
+                               ("stiff", 2, False, "fp64"), ("stiff", 1, True, "fp64"))]
+
+
+@pytest.mark.parametrize("n,kind,rs,per,precision", MORE)
+def test_tile_matches_march_more_forms(gpu, n, kind, rs, per, precision):
+    """Conversions of the stiffened gas cancel 7.8e3 against a pressure of 1, as those of
+    water/air cancel 3e9 against 1e5, and viscous faces divide rounded differences by a
+    cell width: 1e-9 for all of them in FP64."""
+    cfg, mesh, st, eos = _build_more(n, kind, per, precision)
+    ta, a = _fields(cfg, mesh, st, eos, rs, precision, 0)
+    tb, b = _fields(cfg, mesh, st, eos, rs, precision, 8)
+    bar = 2e-5 if precision == "mixed" else 1e-9
+    assert abs(ta - tb) <= bar * tb
+    for f in a:
+        if abs(b[f]).max() > 0.0:
+            assert rel_errs(a[f], b[f])[1] <= bar, (f, rel_errs(a[f], b[f]))
+        else:
+            assert abs(a[f]).max() == 0.0
+
+
+@pytest.mark.parametrize("n", [(62, 8), (63, 9)] + LARGE)
+def test_tile_stiffened_fp32_error(gpu, n):
+    """FP32 star states of a stiffened gas cancel energies of 7.8e3 times a wave speed of
+    160 against a pressure of 1, some 1e-4 of it a stage: tiles and march may differ by as
+    much, but the tiles' error against the FP64 state is that of the march (mean over the
+    cells, within a factor of 1.5)."""
+    cfg, mesh, st, eos = _build_more(n, "stiff", True, "mixed")
+    runs = [_fields(cfg, mesh, st, eos, 2, *form)[1] for form in (("fp64", 8), ("mixed", 0), ("mixed", 8))]
+    for f in runs[0]:
+        if abs(runs[0][f]).max() > 0.0:
+            tile, march = (rel_errs(r[f], runs[0][f])[0] for r in runs[1:])
+            assert tile <= 1.5 * march, (f, tile, march)
+
+
+@pytest.mark.parametrize("n", [(63, 9), (130, 700)])   # 2-row and 8-row tiles
+def test_tile_step_graph(gpu, n):
+    """Every source term on tiles: a replayed step graph gives the launches' bits."""
+    runs = []
+    for graphs in (True, False):
+        cfg, mesh, st, eos = _build_more(n, "two_source", False, "fp64")
+        g = ExplicitSolver(mesh, HLLCSolver(eos), eos, None, cfg)
+        g.set_graphs(graphs)
+        g.upload(st)
+        t = 0.0
+        for k in (3, 4):
+            t, done = g.advance(cfg, k, 1e30, t)
+            assert done == k
+        assert (g.graph_replays() > 0) == graphs
+        runs.append((t, [g.download_field(f).copy() for f in st.field_ids()]))
+        g.close()
+    assert runs[0][0] == runs[1][0]
+    assert all((mesh.interior(x) == mesh.interior(y)).all() for x, y in zip(runs[0][1], runs[1][1]))
+
+
 @pytest.mark.parametrize("rk,recon", [(1, RO.WENO5), (2, RO.UPWIND5), (3, RO.WENO5)])
 @pytest.mark.parametrize("n", [(62, 8), (63, 17), (130, 400)])
 def test_tile_matches_oracle(gpu, oracle_c, n, rk, recon):
