@@ -12,7 +12,7 @@ EXE = os.path.join(ROOT, "oracle", "_ref", "dropin_driver")
 
 
 def test_dropin_driver_was_built():
-    if not os.path.isdir("/root/reference"):
+    if not os.path.isdir("/root/reference/src"):
         pytest.skip("reference checkout absent")
     assert os.path.exists(EXE), "oracle/Makefile did not build the C++ drop-in driver"
 
