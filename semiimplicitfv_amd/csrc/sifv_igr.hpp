@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(64) igr_sweep_kernel(IgrSweepArgs A) {
 // times (ny + 64 W) / 8, and around a wrapping axis the hand-off of every strip
 // (about 8 us beyond the 64 steps).  Microseconds a sweep, one wave with loads,
 // coefficients and sweeps in one and a release / acquire hand-off -> now: 1024^2
-// wrapping 468 -> 251, 1024^2 walls 240 -> 148, 2048^2 981 -> 536 and 580 -> 325.
+// wrapping 468 -> 242, 1024^2 walls 240 -> 144, 2048^2 981 -> 521 and 580 -> 318.
 // Ghost semantics are those of the per-sweep scalar fill: zero-gradient
 // faces read the cell's own previous-sweep value, wrapping y faces the
 // previous result (bottom) and the saved previous-sweep row-0 value (top).

@@ -8,9 +8,9 @@
 // Each row scaled by V/c (V the cell volume) gives
 //     S_ii = V/c + sum_f w_f,   S_i,nb(f) = -w_f,
 //     w_f  = area_f / (max(0.5 (rho_i + rho_nb), 1e-14) * 0.5 (h_i + h_nb)),
-// symmetric positive definite (both rows of a face compute the same w_f; the
-// host refuses periodic axes whose ghost widths differ from the wrapped
-// cells').  Conjugate gradients on S p = (V/c) rhs with the diagonal of S as
+// symmetric positive definite (both rows of a face have the same w_f, from the
+// stored weights bit for bit and from the densities to their last bits; the host
+// refuses periodic axes whose ghost widths differ from the wrapped cells').  Conjugate gradients on S p = (V/c) rhs with the diagonal of S as
 // preconditioner, in the HYPRE_StructPCG role (src/HyprePressureSolver.cpp:
 // 119-138, 350-358); stop when ||rhs - (1 + c L) p||_2 <= tol ||rhs||_2,
 // compared as squares, the original residual being r / (V/c).

@@ -19,7 +19,8 @@
 // below it in LDS, where the x-stencil of the current row is read anyway.
 // (All rows in registers took 176 VGPRs, one wave per SIMD fewer or spills;
 // spilled registers cost HBM traffic.  4096^2 FP64: 843 -> 758 us per launch
-// together with weno5_set and row addressing, same box.)  Each lane
+// together with weno5_set and row addressing, same box.  Two-phase 2D keeps its
+// own cell of the current row in registers too.)  Each lane
 // reconstructs its own cell once per direction (both face states from one
 // stencil), so every face flux is computed once per strip.
 // 3D: the same kernel runs on each z-plane (MODE_XY) and writes the x+y part
